@@ -9,11 +9,27 @@
 // are out of bounds or under the threshold still add to the weight sum; no
 // sRGB encode. UNORM8 conversion: floor(c * 255 + 0.5).
 //
-// The blur is a 1-D stencil: each block stages the row (or column) segment it
-// needs, plus the per-tap weights, in LDS, so HBM sees each input texel once
-// per pass. The weights depend only on the tap offset and are evaluated once
-// per block.
+// The blur's sums run over the taps in order with separate multiplies and
+// adds (the result's bits depend on it), so its cost is 6 VALU operations per
+// tap and pixel. Two kernels:
+//   k_blur_row     blurX: one block per row, the thresholded row staged in LDS
+//   k_blur_column  blurY, combine and tonemap: one lane per column, rows read
+//                  straight from memory (64 columns = 1 KB per load)
+// Both give a lane several neighbouring outputs, so a sample is loaded once
+// for all of them, and take the weights from the kernel arguments (scalar
+// registers). They leave out the taps whose weight is exactly zero: sigma is
+// the percentage, so of the 577 taps of a 1920-pixel row at the default
+// radius only the middle 145 have a weight that FP32 can hold. A zero weight
+// adds nothing to a finite sum; a row or column window holding a non-finite
+// value (zero times which is NaN) sums every tap. 1920x1080, radius 5: blurX
+// 1091 -> 58 us, blurY with combine and tonemap 620 -> 65 us (3.6 G operations
+// of the weighted taps: 46 us each at one per lane and clock); 341x213: 38 ->
+// 16 us.
+// k_blur and k_combine_tonemap, with the taps' weights in LDS, take the sizes
+// those two do not (see launch_postprocess).
 #include <hip/hip_runtime.h>
+
+#include <cmath>
 
 #include "rt_math.h"
 #include "wavefront.h"
@@ -23,7 +39,7 @@ namespace rt {
 constexpr int kTile = 256;        // output pixels per block along the blur axis
 constexpr int kMaxHalf = 1024;    // LDS-staged half-width; larger kernels read HBM directly
 
-__device__ __forceinline__ float gauss(float x, float sigma) { return expf_(((-x) * x) / ((2.0f * sigma) * sigma)); }
+RT_HD float gauss(float x, float sigma) { return expf_(((-x) * x) / ((2.0f * sigma) * sigma)); }
 
 // axis 1 = X (along rows), 0 = Y (along columns)
 template <int AXIS, bool THRESH>
@@ -89,17 +105,11 @@ __device__ __forceinline__ float rrt1(float v) {
 
 __device__ __forceinline__ uint32_t unorm8(float c) { return (uint32_t)f2i_(floorf(c * 255.0f + 0.5f)) & 0xFFu; }
 
-// combine + tonemap fused: the combined image is also written (it is the
-// reference's ping image at that point).
-__global__ __launch_bounds__(256) void k_combine_tonemap(const float4* __restrict__ orig, const float4* __restrict__ bloom,
-                                                         float4* __restrict__ combined, uchar4* __restrict__ out,
-                                                         uint32_t n, float intensity, float exposure) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float4 o = orig[i], bl = bloom[i];
+// combine and tonemap of one pixel; scale = 2^exposure
+__device__ __forceinline__ uchar4 combine_tonemap(float4 o, V3 bl, float intensity, float exposure_scale, float4& combined) {
     V3 c = v3(o.x + bl.x * intensity, o.y + bl.y * intensity, o.z + bl.z * intensity);
-    combined[i] = make_float4(c.x, c.y, c.z, 1.0f);
-    float e = exp2f_(exposure);
+    combined = make_float4(c.x, c.y, c.z, 1.0f);
+    const float e = exposure_scale;
     c = v3(c.x * e, c.y * e, c.z * e);
     c = v3(dot(c, v3(0.59719f, 0.35458f, 0.04823f)), dot(c, v3(0.07600f, 0.90834f, 0.01566f)),
            dot(c, v3(0.02840f, 0.13383f, 0.83777f)));
@@ -107,22 +117,255 @@ __global__ __launch_bounds__(256) void k_combine_tonemap(const float4* __restric
     c = v3(dot(c, v3(1.60475f, -0.53108f, -0.07367f)), dot(c, v3(-0.10208f, 1.10813f, -0.00605f)),
            dot(c, v3(-0.00327f, -0.07276f, 1.07602f)));
     c = v3(clampf_(c.x, 0.0f, 1.0f), clampf_(c.y, 0.0f, 1.0f), clampf_(c.z, 0.0f, 1.0f));
-    out[i] = make_uchar4((unsigned char)unorm8(c.x), (unsigned char)unorm8(c.y), (unsigned char)unorm8(c.z), 255);
+    return make_uchar4((unsigned char)unorm8(c.x), (unsigned char)unorm8(c.y), (unsigned char)unorm8(c.z), 255);
 }
+
+// combine + tonemap fused: the combined image is also written (it is the
+// reference's ping image at that point).
+__global__ __launch_bounds__(256) void k_combine_tonemap(const float4* __restrict__ orig, const float4* __restrict__ bloom,
+                                                         float4* __restrict__ combined, uchar4* __restrict__ out,
+                                                         uint32_t n, float intensity, float exposure_scale) {
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const float4 bl = bloom[i];
+    float4 c;
+    const uchar4 t = combine_tonemap(orig[i], v3(bl.x, bl.y, bl.z), intensity, exposure_scale, c);
+    combined[i] = c;
+    out[i] = t;
+}
+
+// ---- blur over the taps with a weight ----------------------------------------
+constexpr int kTapPad = 16;      // zero weights before the first and after the last tap
+constexpr int kMaxTapHalf = 448; // 3.7 KB of the 4 KB of kernel arguments
+// No sum of samples up to this overflows (the weights add up to 2.51 sigma + 1 at most).
+constexpr float kFinite = 1.0e34f;
+
+// w[kTapPad + i + half] is the weight of tap i, zero outside [-k, k].
+struct Taps {
+    int32_t k;      // the stencil's half-width
+    int32_t half;   // a multiple of 4; every tap beyond it has weight zero
+    float wsum;     // sum over all taps, in tap order
+    float w[2 * kMaxTapHalf + 1 + 2 * kTapPad];
+};
+
+// Adds the taps of samples m0..m0+U-1 to R neighbouring outputs: sample m is
+// tap m - half of output 0, m - 1 - half of output 1, ...
+template <int R, int U>
+__device__ __forceinline__ void add_taps(const Taps& t, int m0, const float (&x)[3][U], float (&c)[R][3]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const float w = t.w[kTapPad + m0 + u - j];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) c[j][a] = c[j][a] + x[a][u] * w;
+        }
+    }
+}
+
+__device__ __forceinline__ V3 blur_mean(const float (&c)[3], float wsum) {
+    return wsum < 0.0001f ? v3(0.0f, 0.0f, 0.0f) : v3(c[0] / wsum, c[1] / wsum, c[2] / wsum);
+}
+
+// blurX of row blockIdx.x. The row's three channels lie in LDS, `half` zeros on
+// either side; a lane's R outputs are neighbours, so R = 4 reads four samples of
+// a channel with one 16-byte load for 16 multiply-adds. out.w is 1, or 2 in a
+// row whose samples are not all finite (or near overflow).
+template <int R, int U>
+__global__ __launch_bounds__(1024) void k_blur_row(const float4* __restrict__ in, float4* __restrict__ out, uint32_t W,
+                                                   uint32_t pitch, float threshold, const Taps t) {
+    extern __shared__ __align__(16) float s_row[];   // [3][pitch]
+    const float4* src = in + (uint64_t)blockIdx.x * W;
+    float4* dst = out + (uint64_t)blockIdx.x * W;
+    bool bad = false;
+    for (uint32_t p = threadIdx.x; p < pitch; p += blockDim.x) {
+        const int32_t x = (int32_t)p - t.half;
+        float r = 0.0f, g = 0.0f, b = 0.0f;
+        if (x >= 0 && x < (int32_t)W) {
+            const float4 v = src[x];
+            if (!(dot(v3(v.x, v.y, v.z), v3(0.299f, 0.587f, 0.114f)) < threshold)) { r = v.x; g = v.y; b = v.z; }
+            bad = bad || !(fabsf(r) <= kFinite && fabsf(g) <= kFinite && fabsf(b) <= kFinite);
+        }
+        s_row[p] = r;
+        s_row[pitch + p] = g;
+        s_row[2 * pitch + p] = b;
+    }
+    const bool every = __syncthreads_or(bad ? 1 : 0) != 0;   // every tap counts
+    for (uint32_t x0 = threadIdx.x * R; x0 < W; x0 += blockDim.x * R) {
+        float c[R][3];
+#pragma unroll
+        for (int j = 0; j < R; ++j) c[j][0] = c[j][1] = c[j][2] = 0.0f;
+        if (!every) {
+            const float* p0 = s_row + x0;
+            for (int m = 0; m < 2 * t.half + R; m += U) {
+                float x[3][U];
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    if constexpr (R == 4) {   // x0, m and pitch are multiples of 4
+#pragma unroll
+                        for (int u = 0; u < U; u += 4) {
+                            const float4 v = *reinterpret_cast<const float4*>(p0 + a * pitch + m + u);
+                            x[a][u] = v.x; x[a][u + 1] = v.y; x[a][u + 2] = v.z; x[a][u + 3] = v.w;
+                        }
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < U; ++u) x[a][u] = p0[a * pitch + m + u];
+                    }
+                }
+                add_taps<R, U>(t, m, x, c);
+            }
+        } else {
+            for (int j = 0; j < R; ++j) {
+                for (int32_t i = -t.k; i <= t.k; ++i) {
+                    const int32_t x = (int32_t)(x0 + j) + i;
+                    if (x < 0 || x >= (int32_t)W) continue;
+                    const float w = (i < -t.half || i > t.half) ? 0.0f : t.w[kTapPad + i + t.half];
+                    const float* p = s_row + x + t.half;
+                    c[j][0] = c[j][0] + p[0] * w;
+                    c[j][1] = c[j][1] + p[pitch] * w;
+                    c[j][2] = c[j][2] + p[2 * pitch] * w;
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            if (x0 + j >= W) break;
+            const V3 v = blur_mean(c[j], t.wsum);
+            dst[x0 + j] = make_float4(v.x, v.y, v.z, every ? 2.0f : 1.0f);
+        }
+    }
+}
+
+// blurY, combine and tonemap of 64 columns x 4 R rows; wave w takes R rows and
+// loads U samples at a time (enough in flight to cover the load's latency).
+template <int R, int U>
+__global__ __launch_bounds__(256) void k_blur_column(const float4* __restrict__ blurx, const float4* __restrict__ orig,
+                                                     float4* __restrict__ combined, uchar4* __restrict__ out, uint32_t W,
+                                                     uint32_t H, float intensity, float exposure_scale, const Taps t) {
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t xb = blockIdx.x * 64u, x = xb + lane;
+    const int32_t yb = (int32_t)(blockIdx.y * 4u * R);
+    // rows that k_blur_row marked, among all that the sums below read: k either
+    // side, and the zero-weight taps up to the next multiple of U
+    const int32_t reach = t.k > t.half + U ? t.k : t.half + U;
+    bool bad = false;
+    for (int32_t y = yb - reach + (int32_t)threadIdx.x; y < yb + 4 * R + reach; y += 256)
+        if (y >= 0 && y < (int32_t)H) bad = bad || blurx[(uint64_t)y * W + xb].w != 1.0f;
+    const bool every = __syncthreads_or(bad ? 1 : 0) != 0;
+    const int32_t y0 = __builtin_amdgcn_readfirstlane(yb + (int32_t)(wave * R));
+    if (x >= W || y0 >= (int32_t)H) return;
+    float c[R][3];
+#pragma unroll
+    for (int j = 0; j < R; ++j) c[j][0] = c[j][1] = c[j][2] = 0.0f;
+    const float4* col = blurx + x;
+    if (!every) {
+        for (int m = 0; m < 2 * t.half + R; m += U) {
+            float s[3][U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int32_t y = y0 - t.half + m + u;
+                float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (y >= 0 && y < (int32_t)H) v = col[(uint64_t)(uint32_t)y * W];
+                s[0][u] = v.x; s[1][u] = v.y; s[2][u] = v.z;
+            }
+            add_taps<R, U>(t, m, s, c);
+        }
+    } else {
+        for (int j = 0; j < R; ++j) {
+            for (int32_t i = -t.k; i <= t.k; ++i) {
+                const int32_t y = y0 + j + i;
+                if (y < 0 || y >= (int32_t)H) continue;
+                const float w = (i < -t.half || i > t.half) ? 0.0f : t.w[kTapPad + i + t.half];
+                const float4 v = col[(uint64_t)(uint32_t)y * W];
+                c[j][0] = c[j][0] + v.x * w;
+                c[j][1] = c[j][1] + v.y * w;
+                c[j][2] = c[j][2] + v.z * w;
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+        if (y0 + j >= (int32_t)H) break;
+        const uint64_t o = (uint64_t)(uint32_t)(y0 + j) * W + x;
+        float4 cm;
+        const uchar4 ldr = combine_tonemap(orig[o], blur_mean(c[j], t.wsum), intensity, exposure_scale, cm);
+        combined[o] = cm;
+        out[o] = ldr;
+    }
+}
+
+// The taps of a blur over `len` pixels; false where k_blur has to do it: a
+// radius that is not positive and finite, or more taps than the kernel
+// arguments hold (radius above 31 on images over 480 pixels).
+static bool make_taps(uint32_t len, float radius, Taps& t) {
+    const float k = ((float)(int32_t)len * radius) / 100.0f * 3.0f + 0.5f;
+    if (!(radius > 0.0f && k >= 0.0f && k < 1.0e6f)) return false;
+    t.k = (int32_t)k;
+    // expf_ returns 0 below -103.97: beyond sqrt(2 * 103.98) sigma nothing is left
+    const float reach = 14.43f * radius + 2.0f;
+    int32_t h = reach < (float)t.k ? (int32_t)reach : t.k;
+    if (h > kMaxTapHalf) return false;
+    float w[kMaxTapHalf + 1];
+    for (int32_t i = 0; i <= h; ++i) w[i] = gauss((float)i, radius);   // even in i
+    while (h > 0 && w[h] == 0.0f) --h;
+    t.half = (h + 3) & ~3;
+    for (int32_t i = 0; i < 2 * t.half + 1 + 2 * kTapPad; ++i) {
+        const int32_t tap = i - kTapPad - t.half, a = tap < 0 ? -tap : tap;
+        t.w[i] = a <= h ? w[a] : 0.0f;
+    }
+    t.wsum = 0.0f;
+    for (int32_t i = -h; i <= h; ++i) t.wsum = t.wsum + w[i < 0 ? -i : i];
+    return true;
+}
+
+template <int R, int U>
+static void launch_blur_row(const float4* in, float4* out, uint32_t W, uint32_t H, uint32_t pitch, float threshold,
+                            const Taps& t, hipStream_t st) {
+    uint32_t threads = ((W + R - 1) / R + 63u) & ~63u;
+    if (threads > 1024u) threads = 1024u;
+    hipLaunchKernelGGL((k_blur_row<R, U>), dim3(H), dim3(threads), 3u * pitch * sizeof(float), st, in, out, W, pitch, threshold, t);
+}
+
+template <int R, int U>
+static void launch_blur_column(const float4* blurx, const float4* orig, float4* combined, uchar4* out, uint32_t W,
+                               uint32_t H, float intensity, float exposure_scale, const Taps& t, hipStream_t st) {
+    hipLaunchKernelGGL((k_blur_column<R, U>), dim3((W + 63) / 64, (H + 4 * R - 1) / (4 * R)), dim3(256), 0, st, blurx, orig,
+                       combined, out, W, H, intensity, exposure_scale, t);
+}
+
+// k_blur_row holds a row in 64 KB of LDS: rows of up to about 5,200 pixels.
+constexpr uint32_t kRowLds = 65536;
 
 hipError_t launch_postprocess(const float4* in, float4* ping, float4* pong, uchar4* out, uint32_t W, uint32_t H,
                               const BloomPushConsts& b, const TonemappingPushConsts& t, hipStream_t st) {
+    const float e = exp2f_(t.exposure);
+    hipError_t err;
+    Taps tx, ty;
+    if (make_taps(W, b.radius, tx) && make_taps(H, b.radius, ty)) {
+        // staged width: the last lane's last group of samples ends at W + 2 half + 16
+        const uint32_t pitch = (W + 2u * (uint32_t)tx.half + 16u + 3u) & ~3u;
+        if (3ull * pitch * sizeof(float) <= kRowLds && (H + 3u) / 4u <= 65535u) {
+            // outputs per lane: as many as leave a few waves for each of the 1,024 SIMDs
+            if ((uint64_t)W * H >= (1u << 19)) launch_blur_row<4, 4>(in, pong, W, H, pitch, b.threshold, tx, st);
+            else launch_blur_row<1, 16>(in, pong, W, H, pitch, b.threshold, tx, st);
+            err = hipGetLastError();
+            if (err != hipSuccess) return err;
+            if ((uint64_t)W * H >= (1u << 19)) launch_blur_column<8, 8>(pong, in, ping, out, W, H, b.intensity, e, ty, st);
+            else launch_blur_column<1, 16>(pong, in, ping, out, W, H, b.intensity, e, ty, st);
+            return hipGetLastError();
+        }
+    }
     dim3 gx((W + kTile - 1) / kTile, H);
     hipLaunchKernelGGL((k_blur<1, true>), gx, dim3(kTile), 0, st, in, ping, W, H, b);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    err = hipGetLastError();
+    if (err != hipSuccess) return err;
     dim3 gy((H + kTile - 1) / kTile, W);
     hipLaunchKernelGGL((k_blur<0, false>), gy, dim3(kTile), 0, st, ping, pong, W, H, b);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    err = hipGetLastError();
+    if (err != hipSuccess) return err;
     uint32_t n = W * H;
     hipLaunchKernelGGL(k_combine_tonemap, dim3((n + 255) / 256), dim3(256), 0, st, in, pong, ping, out, n,
-                       b.intensity, t.exposure);
+                       b.intensity, e);
     return hipGetLastError();
 }
 

@@ -21,6 +21,7 @@
 #include <stdint.h>
 
 #define RT_D __device__ __forceinline__
+#define RT_HD __host__ __device__ __forceinline__   // the same operations on the host, bit for bit
 
 namespace rt {
 
@@ -86,9 +87,9 @@ RT_D float logf_(float x) {
     return dk * 0.693145751953125f - ((hfsq - (s * (hfsq + R) + dk * 1.4286068e-06f)) - f);
 }
 
-RT_D float pow2i_(int j) { return __uint_as_float((uint32_t)(j + 127) << 23); }
+RT_HD float pow2i_(int j) { return __builtin_bit_cast(float, (uint32_t)(j + 127) << 23); }
 
-RT_D float exp_tail(float r, float kf) {
+RT_HD float exp_tail(float r, float kf) {
     float p = 2.4801587e-5f;
     p = p * r + 1.9841270e-4f;
     p = p * r + 1.3888889e-3f;
@@ -104,7 +105,7 @@ RT_D float exp_tail(float r, float kf) {
     return (p * pow2i_(k1)) * pow2i_(k2);
 }
 
-RT_D float expf_(float x) {
+RT_HD float expf_(float x) {
     if (x != x) return x;
     if (x > 88.72283f) return __builtin_inff();
     if (x < -103.97208f) return 0.0f;
@@ -113,7 +114,7 @@ RT_D float expf_(float x) {
     return exp_tail(r, kf);
 }
 
-RT_D float exp2f_(float x) {
+RT_HD float exp2f_(float x) {
     if (x != x) return x;
     if (x > 128.0f) return __builtin_inff();
     if (x < -150.0f) return 0.0f;

@@ -1,0 +1,50 @@
+"""Bloom and tone mapping: the per-row and per-column kernels (and the kernels
+that take the sizes those do not) equal the oracle's restatement bit for bit
+over sizes at the edges of their tiles, radii and non-finite samples."""
+import numpy as np
+import pytest
+
+import oracle
+import reina_rt
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(torch, img, radius, threshold):
+    H, W = img.shape[:2]
+    ref_out, ref_comb = oracle.postprocess(img, radius=radius, threshold=threshold, intensity=0.25, exposure=0.5)
+    t_in = torch.from_numpy(img).cuda()
+    scratch = torch.full((2, H, W, 4), float("nan"), device="cuda")
+    out = torch.zeros((H, W, 4), dtype=torch.uint8, device="cuda")
+    reina_rt.postprocess(t_in.data_ptr(), scratch.data_ptr(), out.data_ptr(), W, H, radius, threshold, 0.25, 0.5)
+    torch.cuda.synchronize()
+    comb = scratch[0].cpu().numpy()
+    same = (comb.view(np.uint32) == ref_comb.view(np.uint32)) | (np.isnan(comb) & np.isnan(ref_comb))
+    assert same.all()
+    assert np.array_equal(out.cpu().numpy(), ref_out)
+
+
+# radius 5: half-widths k from 0 (4 pixels and fewer) past the last tap with a
+# weight (72: images over 480 pixels); 40 on 500 pixels: more taps than the
+# kernel arguments hold; 5300 pixels: rows longer than the staged LDS row
+@pytest.mark.parametrize("W,H,radius", [(1, 1, 5.0), (3, 2, 5.0), (63, 5, 5.0), (64, 9, 5.0), (65, 33, 0.7),
+                                        (257, 31, 5.0), (487, 3, 5.0), (1023, 513, 5.0), (1030, 521, 2.0), (60, 700, 5.0),
+                                        (500, 7, 40.0), (5300, 3, 1.0)])
+def test_postprocess_sizes_bitexact(cuda, W, H, radius):
+    rng = np.random.default_rng(W * 1000 + H)
+    img = (rng.random((H, W, 4)) ** 4 * 4.0 - 0.1).astype(np.float32)
+    img[..., 3] = 1.0
+    _check(cuda, img, radius, 1.0)
+
+
+# 700 x 800 takes several outputs per lane, 600 x 90 one
+@pytest.mark.parametrize("W,H", [(700, 800), (600, 90)])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf, 3.0e38])
+def test_postprocess_non_finite_bitexact(cuda, W, H, value):
+    """A sample that is not finite reaches every pixel within the stencil's
+    half-width, also where its weight is zero (0 * inf and 0 * NaN are NaN)."""
+    rng = np.random.default_rng(5)
+    img = rng.random((H, W, 4)).astype(np.float32)
+    img[H // 3, W // 4, 1] = value
+    img[H // 3, W // 4 + 1, 0] = value
+    _check(cuda, img, 5.0, 0.5)
