@@ -107,6 +107,33 @@ static int validate(const ReinaSceneDesc* d) {
     return REINA_RT_OK;
 }
 
+// The inverse transpose of the instance's 3x3 matrix by its cofactors, in the
+// operation order of closestHitCommon.h.glsl:110-112's restatement.
+static void set_normal_matrix(InstanceRec& r) {
+    const V3 c0 = v3(r.c0[0], r.c0[1], r.c0[2]), c1 = v3(r.c1[0], r.c1[1], r.c1[2]), c2 = v3(r.c2[0], r.c2[1], r.c2[2]);
+    const float invdet = 1.0f / dot(c0, cross(c1, c2));
+    const V3 n[3] = {scale(cross(c1, c2), invdet), scale(cross(c2, c0), invdet), scale(cross(c0, c1), invdet)};
+    float* out[3] = {r.n0, r.n1, r.n2};
+    for (int k = 0; k < 3; ++k) { out[k][0] = n[k].x; out[k][1] = n[k].y; out[k][2] = n[k].z; }
+    r.pad[0] = r.pad[1] = r.pad[2] = 0.0f;
+}
+
+// The operations of evalDisney's and sampleDisney's weights and GGX alphas
+// (shade.h), which depend on the properties alone.
+static MaterialRec make_material(const ReinaInstanceProperties& p) {
+    MaterialRec m{};
+    alphas(p.anisotropic, p.roughness, m.ax, m.ay);
+    const float st = p.specularTransmission, dW = (1.0f - st) * (1.0f - p.metallic), gW = (1.0f - p.metallic) * st;
+    m.ws = (dW + p.metallic) + gW;
+    m.dWn = dW / m.ws;
+    m.mWn = p.metallic / m.ws;
+    m.gWn = gW / m.ws;
+    const float ag = clearcoat_alpha(p.clearcoatGloss);
+    m.dcn = ag * ag - 1.0f;
+    m.dcl = kPi * logf_(ag * ag);
+    return m;
+}
+
 // Light-sampling tables (EmissiveInst, rt_layout.h) from the flattened
 // world-space triangles, in double precision.
 static void build_emissive(ReinaScene* s, const ReinaSceneDesc* d, const std::vector<InstanceRec>& inst,
@@ -180,6 +207,9 @@ static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vecto
     size_t p_tp = add(tri_prim.data(), tri_prim.size() * 4);
     size_t p_in = add(inst.data(), inst.size() * sizeof(InstanceRec));
     size_t p_pr = add(d->props, (uint64_t)d->num_props * sizeof(ReinaInstanceProperties));
+    std::vector<MaterialRec> mats(d->num_props);
+    for (uint32_t i = 0; i < d->num_props; ++i) mats[i] = make_material(d->props[i]);
+    size_t p_mat = add(mats.data(), mats.size() * sizeof(MaterialRec));
     size_t p_v = add(d->vertices, d->num_vertices * 16);
     size_t p_i = add(d->indices, d->num_indices * 4);
     size_t p_t = add(d->tbns, d->num_tbns * 36);
@@ -218,6 +248,7 @@ static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vecto
     s->sv.tri_prim = (const uint32_t RT_GLOBAL*)(a + parts[p_tp].off);
     s->sv.inst = (const InstanceRec RT_GLOBAL*)(a + parts[p_in].off);
     s->sv.props = (const ReinaInstanceProperties RT_GLOBAL*)(a + parts[p_pr].off);
+    s->sv.mats = (const MaterialRec RT_GLOBAL*)(a + parts[p_mat].off);
     s->sv.vertices = (const float4 RT_GLOBAL*)(a + parts[p_v].off);
     s->sv.indices = (const uint32_t RT_GLOBAL*)(a + parts[p_i].off);
     s->sv.tbns = (const float RT_GLOBAL*)(a + parts[p_t].off);
@@ -267,6 +298,7 @@ int reina_rt_scene_create(const ReinaSceneDesc* d, ReinaScene** out) {
         r.material = id.materialIdx;
         r.model = id.modelID;
         r.tri_base = (uint32_t)ntri;
+        set_normal_matrix(r);
         ntri += d->models[id.modelID].indexCount;
     }
     if (ntri >= (1ull << 24)) return fail(REINA_RT_ERR_INVALID_ARG, "more than 2^24 triangles in one scene");

@@ -37,6 +37,8 @@ inline TraceParams make_trace_params(const RtPushConsts* pc, uint32_t W, uint32_
     P.cam.defocus = pc->defocusMultiplier;
     P.cam.W = (float)(int32_t)W;
     P.cam.H = (float)(int32_t)H;
+    P.cam.right = normalize(v3(pc->invView[0], pc->invView[1], pc->invView[2]));
+    P.cam.up = normalize(v3(pc->invView[4], pc->invView[5], pc->invView[6]));
     P.W = W;
     P.H = H;
     P.spp = pc->samplesPerPixel;

@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void k_init(TraceParams P, PathState S, Queues
 // tiles of 256 rays, and the survivors of a tile are appended to the same
 // partition of the next queue with one atomic (wave ballot + LDS scan).
 template <bool NEE>
-__global__ __launch_bounds__(256) void k_shade(SceneView sv, TraceParams P, PathState S, Queues Q, uint32_t in_q,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NEE ? 0 : 3))) void k_shade(SceneView sv, TraceParams P, PathState S, Queues Q, uint32_t in_q,
                                                Ctrl* ctrl, uint32_t slot) {
     __shared__ uint32_t s_wave[4];
     __shared__ uint32_t s_base;

@@ -78,15 +78,30 @@ constexpr float kCollapseTriCost = 0.5f;
 
 // Triangles in leaf order: 3 x float4 = (v0.xyz, id bits), (v1.xyz, 0), (v2.xyz, 0).
 
-// Per-instance record used by the shading kernels (64 bytes).
+// Per-instance record used by the shading kernels (112 bytes; the first 64
+// serve every hit, the normal matrix only those that need a tangent frame).
 struct alignas(16) InstanceRec {
     float c0[3], c1[3], c2[3], c3[3];   // gl_ObjectToWorldEXT columns
     uint32_t props_id;
     uint32_t material;
     uint32_t model;
     uint32_t tri_base;                  // first flattened triangle id
+    float n0[3], n1[3], n2[3];          // columns of the inverse transpose of (c0, c1, c2)
+    float pad[3];
 };
-static_assert(sizeof(InstanceRec) == 64, "instance record size");
+static_assert(sizeof(InstanceRec) == 112, "instance record size");
+
+// What the Disney hit shader derives from one InstanceProperties record alone,
+// worked out once per scene instead of at every hit (evalDisney and
+// sampleDisney as the reference weights them; the corrected mixture of
+// REINA_RT_TRACE_FIX_DISNEY_MIX divides by its own sum).
+struct alignas(16) MaterialRec {
+    float ax, ay;            // GGX alphas
+    float ws;                // diffuse + metal + glass weight
+    float dWn, mWn, gWn;     // those weights over ws
+    float dcn, dcl;          // clearcoat GTR1: a^2 - 1 and pi log(a^2), a from clearcoatGloss
+};
+static_assert(sizeof(MaterialRec) == 32, "material record size");
 
 // Light sampling for next-event estimation: one record per emissive instance
 // (emission with |e|^2 > 1e-10, src/scene/Instance.cpp:75-77). Instances are
@@ -126,6 +141,7 @@ struct SceneView {
     const uint32_t RT_GLOBAL* tri_prim;    // flattened id -> gl_PrimitiveID
     const InstanceRec RT_GLOBAL* inst;
     const ReinaInstanceProperties RT_GLOBAL* props;
+    const MaterialRec RT_GLOBAL* mats;     // one per props record
     const float4 RT_GLOBAL* vertices;
     const uint32_t RT_GLOBAL* indices;
     const float RT_GLOBAL* tbns;
@@ -144,16 +160,19 @@ struct SceneView {
     const uint8_t RT_GLOBAL* tri_flags;
     uint32_t num_emi;
     uint32_t num_inst;
-    // shading record of flattened triangle g, kShadeRecF4 float4 at srec + kShadeRecF4 * g:
-    // (v0.xyz, instance), (v1.xyz, primitive), (v2.xyz, properties index), then T, B, N of
-    // vertex 0, 1, 2 (27 floats, 1 pad): the object-space values hit_info reads, gathered
-    // once per scene
+    // shading record of flattened triangle g, kShadeRecF4 float4 at srec + kShadeRecF4 * g: the
+    // object-space values hit_info reads and the normals that depend on the triangle alone,
+    // gathered once per scene. A hit loads only what its surface uses:
+    //   0-3   (v0.xyz, instance), (v1.xyz, primitive), (v2.xyz, properties index),
+    //         (world normal of the flat triangle, f[0])                     every hit
+    //   4-6   unit normals of vertex 0, 1, 2, (f[1]), (f[2]), (f[3])        interpolated normals
+    //   7-12  f[4..26], 1 pad; f = T, B, N of vertex 0, 1, 2 as given       tangent frames
     const float4 RT_GLOBAL* srec;
     // textures of InstanceProperties.textureID / normalMapTexID / bumpMapTexID
     const TexInfo RT_GLOBAL* tex;
     const uint32_t RT_GLOBAL* texels;
     uint32_t num_tex;
 };
-constexpr uint32_t kShadeRecF4 = 10;   // 160 bytes
+constexpr uint32_t kShadeRecF4 = 13;   // 208 bytes
 
 }  // namespace rt

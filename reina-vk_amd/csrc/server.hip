@@ -86,7 +86,7 @@ __global__ __launch_bounds__(256) void k_init_job(const JobRec* jobs, uint32_t j
 // present in the wave). NEE: the server holds shadow queues; requests with
 // TraceParams.nee write their shadow rays, every other entry an empty one.
 template <bool NEE>
-__global__ __launch_bounds__(256) void k_shade_multi(const JobRec* jobs, PathState S, Queues Q, uint32_t in_q,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NEE ? 0 : 3))) void k_shade_multi(const JobRec* jobs, PathState S, Queues Q, uint32_t in_q,
                                                      Ctrl* ctrl, uint32_t slot, uint32_t* done) {
     __shared__ uint32_t s_wave[4];
     __shared__ uint32_t s_base;

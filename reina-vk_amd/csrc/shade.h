@@ -30,9 +30,8 @@ struct Payload {
 
 struct HitInfo {
     V3 worldPosition, worldNormal, worldNormalGeometry;
-    float uvx, uvy;
+    float bx, by, bz;   // barycentric weights of vertex 0, 1, 2
     bool frontFace;
-    M3 tbn;
 };
 
 RT_D V3 ldv3(const float* p) { return v3(p[0], p[1], p[2]); }
@@ -46,17 +45,19 @@ RT_D V3 tbn_col(const SceneView& sv, uint32_t pos, int col) {
 
 // The shading record of flattened triangle g (SceneView::srec): the same
 // loads as closestHitCommon.h.glsl:52-148 makes through the instance's index
-// and TBN offsets, done once per scene.
+// and TBN offsets, and the flat triangle's world normal (:58-70, 113-114) and
+// unit vertex normals (:75-77), done once per scene.
 RT_D void shade_record(const SceneView& sv, uint32_t g, float4* r) {
     const uint32_t ii = sv.tri_inst[g], prim = sv.tri_prim[g];
-    const InstanceRec in = sv.inst[ii];
-    const ReinaInstanceProperties& p = sv.props[in.props_id];
+    const InstanceRec RT_GLOBAL& in = sv.inst[ii];
+    const ReinaInstanceProperties RT_GLOBAL& p = sv.props[in.props_id];
     const uint32_t io = p.indicesOffset, to = p.tbnsIndicesOffset;
     float f[28];
+    V3 v[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const float4 v = sv.vertices[sv.indices[3u * prim + io + k]];
-        r[k] = make_float4(v.x, v.y, v.z, __uint_as_float(k == 0 ? ii : (k == 1 ? prim : in.props_id)));
+        const float4 q = sv.vertices[sv.indices[3u * prim + io + k]];
+        v[k] = v3(q.x, q.y, q.z);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             const V3 col = tbn_col(sv, 3u * prim + to + k, c);
@@ -66,69 +67,104 @@ RT_D void shade_record(const SceneView& sv, uint32_t g, float4* r) {
         }
     }
     f[27] = 0.0f;
+    M3 M;
+    M.c0 = v3(in.c0[0], in.c0[1], in.c0[2]);
+    M.c1 = v3(in.c1[0], in.c1[1], in.c1[2]);
+    M.c2 = v3(in.c2[0], in.c2[1], in.c2[2]);
+    const V3 ng = normalize(mmul(M, normalize(cross(sub(v[1], v[0]), sub(v[2], v[0])))));
+    r[0] = make_float4(v[0].x, v[0].y, v[0].z, __uint_as_float(ii));
+    r[1] = make_float4(v[1].x, v[1].y, v[1].z, __uint_as_float(prim));
+    r[2] = make_float4(v[2].x, v[2].y, v[2].z, __uint_as_float(in.props_id));
+    r[3] = make_float4(ng.x, ng.y, ng.z, f[0]);
 #pragma unroll
-    for (int q = 0; q < 7; ++q) r[3 + q] = make_float4(f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]);
+    for (int k = 0; k < 3; ++k) {
+        const V3 n = normalize(v3(f[9 * k + 6], f[9 * k + 7], f[9 * k + 8]));
+        r[4 + k] = make_float4(n.x, n.y, n.z, f[1 + k]);
+    }
+#pragma unroll
+    for (int q = 0; q < 6; ++q) r[7 + q] = make_float4(f[4 + 4 * q], f[5 + 4 * q], f[6 + 4 * q], f[7 + 4 * q]);
 }
 
-// closestHitCommon.h.glsl:52-148, from the triangle's shading record
+RT_D M3 normal_matrix(const InstanceRec RT_GLOBAL& in) {
+    M3 m;
+    m.c0 = v3(in.n0[0], in.n0[1], in.n0[2]);
+    m.c1 = v3(in.n1[0], in.n1[1], in.n1[2]);
+    m.c2 = v3(in.n2[0], in.n2[1], in.n2[2]);
+    return m;
+}
+
+// closestHitCommon.h.glsl:52-118, from the triangle's shading record
 // fix_normals: world normals by the inverse-transpose (REINA_RT_TRACE_FIX_NORMALS)
-RT_D HitInfo hit_info(const SceneView& sv, const InstanceRec& in, const ReinaInstanceProperties& p,
-                      const float4* rec, uint32_t prim, float bu, float bv, V3 D, bool fix_normals) {
+RT_D HitInfo hit_info(const InstanceRec RT_GLOBAL& in, bool interp, const float4 RT_GLOBAL* rec, const float4 (&q)[4],
+                      float bu, float bv, V3 D, bool fix_normals) {
     HitInfo r;
-    float4 q[kShadeRecF4];
-#pragma unroll
-    for (int k = 0; k < (int)kShadeRecF4; ++k) q[k] = rec[k];
-    float tb[28];
-#pragma unroll
-    for (int k = 0; k < 7; ++k) { tb[4 * k] = q[3 + k].x; tb[4 * k + 1] = q[3 + k].y; tb[4 * k + 2] = q[3 + k].z; tb[4 * k + 3] = q[3 + k].w; }
-    // T, B, N of vertex k: tb[9k + 0..2], tb[9k + 3..5], tb[9k + 6..8]
-    V3 v0 = v3(q[0].x, q[0].y, q[0].z), v1 = v3(q[1].x, q[1].y, q[1].z), v2 = v3(q[2].x, q[2].y, q[2].z);
-    float bx = (1.0f - bu) - bv, by = bu, bz = bv;
-    V3 op = add(add(scale(v0, bx), scale(v1, by)), scale(v2, bz));
-    V3 c0 = ldv3(in.c0), c1 = ldv3(in.c1), c2 = ldv3(in.c2), c3 = ldv3(in.c3);
-    r.worldPosition = add(add(add(scale(c0, op.x), scale(c1, op.y)), scale(c2, op.z)), c3);
-    V3 ong = normalize(cross(sub(v1, v0), sub(v2, v0)));
-    V3 on;
-    if (!p.interpNormals) {
-        on = ong;
-    } else {
-        V3 n0 = normalize(v3(tb[6], tb[7], tb[8]));
-        V3 n1 = normalize(v3(tb[15], tb[16], tb[17]));
-        V3 n2 = normalize(v3(tb[24], tb[25], tb[26]));
-        on = normalize(add(add(scale(n0, bx), scale(n1, by)), scale(n2, bz)));
-    }
-    if (p.texIndicesOffset == 0xFFFFFFFFu) {
-        r.uvx = 0.0f; r.uvy = 0.0f;
-    } else {
-        uint32_t tio = p.texIndicesOffset;
-        float tu[3], tv[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            uint32_t ti = sv.tex_indices[3u * prim + tio + k];
-            bool ok = (uint64_t)ti < sv.num_tex_coords;   // 0xFFFFFFFF entries read as (0, 0)
-            tu[k] = ok ? sv.tex_coords[2ull * ti] : 0.0f;
-            tv[k] = ok ? sv.tex_coords[2ull * ti + 1] : 0.0f;
-        }
-        r.uvx = (tu[0] * bx + tu[1] * by) + tu[2] * bz;
-        r.uvy = (tv[0] * bx + tv[1] * by) + tv[2] * bz;
-    }
+    const V3 v0 = v3(q[0].x, q[0].y, q[0].z), v1 = v3(q[1].x, q[1].y, q[1].z), v2 = v3(q[2].x, q[2].y, q[2].z);
+    const float bx = (1.0f - bu) - bv, by = bu, bz = bv;
+    r.bx = bx; r.by = by; r.bz = bz;
+    const V3 op = add(add(scale(v0, bx), scale(v1, by)), scale(v2, bz));
     M3 M;
-    M.c0 = c0; M.c1 = c1; M.c2 = c2;
-    float det = dot(M.c0, cross(M.c1, M.c2));
-    float invdet = 1.0f / det;
-    M3 Ni;
-    Ni.c0 = scale(cross(M.c1, M.c2), invdet);
-    Ni.c1 = scale(cross(M.c2, M.c0), invdet);
-    Ni.c2 = scale(cross(M.c0, M.c1), invdet);
-    const M3& NM = fix_normals ? Ni : M;
-    r.worldNormal = normalize(mmul(NM, on));
-    r.worldNormalGeometry = normalize(mmul(NM, ong));
-    r.frontFace = dot(D, r.worldNormalGeometry) < 0.0f;
-    r.worldNormal = faceforward(r.worldNormal, D, r.worldNormalGeometry);
-    r.worldNormalGeometry = faceforward(r.worldNormalGeometry, D, r.worldNormalGeometry);
-    // TBN, read even when interpNormals is false (closestHitCommon.h.glsl:120-145)
+    M.c0 = v3(in.c0[0], in.c0[1], in.c0[2]);
+    M.c1 = v3(in.c1[0], in.c1[1], in.c1[2]);
+    M.c2 = v3(in.c2[0], in.c2[1], in.c2[2]);
+    const V3 c3 = v3(in.c3[0], in.c3[1], in.c3[2]);
+    r.worldPosition = add(add(add(scale(M.c0, op.x), scale(M.c1, op.y)), scale(M.c2, op.z)), c3);
+    V3 ng = v3(q[3].x, q[3].y, q[3].z), wn = ng;
+    if (fix_normals) {
+        const M3 NM = normal_matrix(in);
+        ng = normalize(mmul(NM, normalize(cross(sub(v1, v0), sub(v2, v0)))));
+        wn = ng;
+        M = NM;
+    }
+    if (interp) {
+        const float4 a = rec[4], b = rec[5], c = rec[6];
+        const V3 on = normalize(add(add(scale(v3(a.x, a.y, a.z), bx), scale(v3(b.x, b.y, b.z), by)),
+                                    scale(v3(c.x, c.y, c.z), bz)));
+        wn = normalize(mmul(M, on));
+    }
+    r.frontFace = dot(D, ng) < 0.0f;
+    r.worldNormal = faceforward(wn, D, ng);
+    r.worldNormalGeometry = faceforward(ng, D, ng);
+    return r;
+}
+
+// closestHitCommon.h.glsl:80-93
+RT_D void hit_uv(const SceneView& sv, const ReinaInstanceProperties& p, uint32_t prim, const HitInfo& hi, float& u,
+                 float& v) {
+    u = 0.0f;
+    v = 0.0f;
+    if (p.texIndicesOffset == 0xFFFFFFFFu) return;
+    const uint32_t tio = p.texIndicesOffset;
+    float tu[3], tv[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        uint32_t ti = sv.tex_indices[3u * prim + tio + k];
+        bool ok = (uint64_t)ti < sv.num_tex_coords;   // 0xFFFFFFFF entries read as (0, 0)
+        tu[k] = ok ? sv.tex_coords[2ull * ti] : 0.0f;
+        tv[k] = ok ? sv.tex_coords[2ull * ti + 1] : 0.0f;
+    }
+    u = (tu[0] * hi.bx + tu[1] * hi.by) + tu[2] * hi.bz;
+    v = (tv[0] * hi.bx + tv[1] * hi.by) + tv[2] * hi.bz;
+}
+
+// The tangent frame, closestHitCommon.h.glsl:120-145. Read only by the Disney
+// shader, normal maps and bump maps: about 9 of a hit's 15 normalisations and
+// 112 of its 208 record bytes, which the other surfaces leave out.
+RT_D M3 hit_tbn(const InstanceRec RT_GLOBAL& in, const float4 RT_GLOBAL* rec, float f0, const HitInfo& hi) {
+    float tb[28];
+    tb[0] = f0;
+    tb[1] = rec[4].w; tb[2] = rec[5].w; tb[3] = rec[6].w;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const float4 q = rec[7 + k];
+        tb[4 * k + 4] = q.x; tb[4 * k + 5] = q.y; tb[4 * k + 6] = q.z; tb[4 * k + 7] = q.w;
+    }
+    // T, B, N of vertex k: tb[9k + 0..2], tb[9k + 3..5], tb[9k + 6..8]
+    M3 M;
+    M.c0 = v3(in.c0[0], in.c0[1], in.c0[2]);
+    M.c1 = v3(in.c1[0], in.c1[1], in.c1[2]);
+    M.c2 = v3(in.c2[0], in.c2[1], in.c2[2]);
     V3 T = v3(0.0f, 0.0f, 0.0f), B = T, N = T;
-    const float w3[3] = {bx, by, bz};
+    const float w3[3] = {hi.bx, hi.by, hi.bz};
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         V3 tk = v3(tb[9 * k], tb[9 * k + 1], tb[9 * k + 2]);
@@ -137,16 +173,16 @@ RT_D HitInfo hit_info(const SceneView& sv, const InstanceRec& in, const ReinaIns
         if (k == 0) { T = scale(tk, w3[0]); B = scale(bk, w3[0]); N = scale(nk, w3[0]); }
         else { T = add(T, scale(tk, w3[k])); B = add(B, scale(bk, w3[k])); N = add(N, scale(nk, w3[k])); }
     }
-    V3 tangent = normalize(T), bitangent = normalize(B), normal = normalize(N);
-    V3 wT = normalize(mmul(M, tangent));
-    V3 wB = normalize(mmul(M, bitangent));
-    V3 wN = normalize(mmul(Ni, normal));
+    V3 wT = normalize(mmul(M, normalize(T)));
+    V3 wB = normalize(mmul(M, normalize(B)));
+    V3 wN = normalize(mmul(normal_matrix(in), normalize(N)));
     wT = normalize(sub(wT, scale(wN, dot(wN, wT))));
     wB = normalize(sub(wB, scale(wN, dot(wN, wB))));
     wB = scale(wB, -1.0f);
-    wN = scale(wN, r.frontFace ? 1.0f : -1.0f);
-    r.tbn.c0 = wT; r.tbn.c1 = wB; r.tbn.c2 = wN;
-    return r;
+    wN = scale(wN, hi.frontFace ? 1.0f : -1.0f);
+    M3 t;
+    t.c0 = wT; t.c1 = wB; t.c2 = wN;
+    return t;
 }
 
 // closestHitCommon.h.glsl:156-177: integer ULP offset, float fallback near 0.
@@ -308,35 +344,38 @@ RT_D float smith_g(V3 wl, float ax, float ay) {                             // :
     return 1.0f / (1.0f + (st - 1.0f) / 2.0f);
 }
 
-RT_D void alphas(float anisotropic, float roughness, float& ax, float& ay) {
+RT_HD void alphas(float anisotropic, float roughness, float& ax, float& ay) {
     float aspect = sqrtf_(1.0f - 0.9f * anisotropic);
     ax = maxf_(0.0001f, (roughness * roughness) / aspect);
     ay = maxf_(0.0001f, (roughness * roughness) * aspect);
 }
 
-RT_D V3 eval_metal(const M3& tbn, V3 bc, float anisotropic, float roughness, V3 n, V3 wi, V3 wo, V3 h,
-                   float specular, V3 specularTint, float metallic, float eta) {   // :247-267
-    float ax, ay;
-    alphas(anisotropic, roughness, ax, ay);
-    V3 fm = eval_fm(bc, h, wo, specular, specularTint, metallic, eta);
+// evalMetal (:247-267) without its Fresnel factor: the distribution, masking
+// and denominator that the metal lobe and the glass lobe's reflection share.
+// All three are even in h, so the glass lobe's flip of h onto n's side changes
+// no bit of them.
+struct GgxTerms {
+    float dm, gm, den;
+};
+RT_D GgxTerms metal_terms(const M3& tbn, float ax, float ay, V3 n, V3 wi, V3 wo, V3 h) {
+    GgxTerms t;
     V3 wiT = normalize(tmul(tbn, wi)), woT = normalize(tmul(tbn, wo)), hT = normalize(tmul(tbn, h));
-    float dm = eval_dm(hT, ax, ay);
-    float gm = smith_g(wiT, ax, ay) * smith_g(woT, ax, ay);
-    float den = (4.0f * fabsf(dot(n, wi))) * fabsf(dot(n, wo));
-    return v3(((fm.x * dm) * gm) / den, ((fm.y * dm) * gm) / den, ((fm.z * dm) * gm) / den);
+    t.dm = eval_dm(hT, ax, ay);
+    t.gm = smith_g(wiT, ax, ay) * smith_g(woT, ax, ay);
+    t.den = (4.0f * fabsf(dot(n, wi))) * fabsf(dot(n, wo));
+    return t;
+}
+RT_D V3 metal_value(V3 fm, const GgxTerms& t) {
+    return v3(((fm.x * t.dm) * t.gm) / t.den, ((fm.y * t.dm) * t.gm) / t.den, ((fm.z * t.dm) * t.gm) / t.den);
 }
 
-RT_D V3 sample_metal(const M3& tbn, float anisotropic, float roughness, V3 wi, uint32_t& rng) {   // :269-285
-    float ax, ay;
-    alphas(anisotropic, roughness, ax, ay);
+RT_D V3 sample_metal(const M3& tbn, float ax, float ay, V3 wi, uint32_t& rng) {   // :269-285
     V3 h = sample_ggx_vndf(tmul(tbn, wi), ax, ay, rng);
     h = normalize(mmul(tbn, h));
     return reflect(neg(wi), h);
 }
 
-RT_D float pdf_metal(const M3& tbn, V3 wi, V3 wo, float anisotropic, float roughness, bool bounded) {   // :287-299
-    float ax, ay;
-    alphas(anisotropic, roughness, ax, ay);
+RT_D float pdf_metal(const M3& tbn, V3 wi, V3 wo, float ax, float ay, bool bounded) {   // :287-299
     return pdf_ggx_reflection(tmul(tbn, wi), tmul(tbn, wo), ax, ay, bounded);
 }
 
@@ -345,34 +384,33 @@ RT_D float g1c(V3 w, float a) {                                             // :
     return 2.0f / (1.0f + sqrtf_(a2 + ((1.0f - a2) * w.z) * w.z));
 }
 
-RT_D float eval_dc(float ag, V3 hl) {                                       // :328-333
-    float num = ag * ag - 1.0f;
-    float den = (kPi * logf_(ag * ag)) * (1.0f + (ag * ag - 1.0f) * (hl.z * hl.z));
-    return num / den;
+// mr.dcn, mr.dcl: the terms of the clearcoat gloss alone
+RT_D float eval_dc(const MaterialRec& mr, V3 hl) {                         // :328-333
+    float den = mr.dcl * (1.0f + mr.dcn * (hl.z * hl.z));
+    return mr.dcn / den;
 }
+RT_HD float clearcoat_alpha(float cg) { return (1.0f - cg) * 0.1f + cg * 0.001f; }
 
-RT_D V3 eval_clearcoat(const M3& tbn, V3 wi, V3 wo, float cg, V3 h) {      // :335-354
-    float ag = (1.0f - cg) * 0.1f + cg * 0.001f;
+RT_D V3 eval_clearcoat(const M3& tbn, V3 wi, V3 wo, const MaterialRec& mr, V3 h) {      // :335-354
     V3 hT = tmul(tbn, h), wiT = tmul(tbn, wi), woT = tmul(tbn, wo);
     float r0 = eval_r0(1.5f);
     float fc = r0 + (1.0f - r0) * pow5_(1.0f - dot(h, wo));
     float gc = g1c(wiT, 0.25f) * g1c(woT, 0.25f);
-    float v = ((0.25f * fc) * gc) * eval_dc(ag, hT);
+    float v = ((0.25f * fc) * gc) * eval_dc(mr, hT);
     return v3(v, v, v);
 }
 
 RT_D V3 sample_clearcoat(const M3& tbn, float cg, V3 wi, uint32_t& rng) {  // :356-366
-    float ag = (1.0f - cg) * 0.1f + cg * 0.001f;
+    float ag = clearcoat_alpha(cg);
     V3 h = normalize(sample_gtr1(ag, rng));
     h = normalize(mmul(tbn, h));
     return normalize(reflect(neg(wi), h));
 }
 
-RT_D float pdf_clearcoat(const M3& tbn, V3 wi, V3 wo, V3 h, float cg) {    // :368-383
-    float ag = (1.0f - cg) * 0.1f + cg * 0.001f;
+RT_D float pdf_clearcoat(const M3& tbn, V3 wi, V3 wo, V3 h, const MaterialRec& mr) {    // :368-383
     V3 wiT = tmul(tbn, wi), woT = tmul(tbn, wo), hT = tmul(tbn, h);
     if (wiT.z <= 0.0f || woT.z <= 0.0f) return 0.0f;
-    float dc = eval_dc(ag, hT) * hT.z;
+    float dc = eval_dc(mr, hT) * hT.z;
     return dc / (4.0f * fabsf(dot(woT, hT)));
 }
 
@@ -383,10 +421,8 @@ RT_D float reflectance(float cosine, float ri) {
     return r0 + (1.0f - r0) * pow5_(1.0f - cosine);
 }
 
-RT_D V3 sample_glass(const M3& tbn, V3 wi, float roughness, float anisotropic, float eta, uint32_t& rng,
+RT_D V3 sample_glass(const M3& tbn, V3 wi, float ax, float ay, float eta, uint32_t& rng,
                      bool& refracted) {                                     // :396-431
-    float ax, ay;
-    alphas(anisotropic, roughness, ax, ay);
     V3 wiT = tmul(tbn, wi);
     V3 hT = sample_ggx_vndf(wiT, ax, ay, rng);
     float cosTheta = dot(wiT, hT);
@@ -407,10 +443,8 @@ RT_D float smith_g_aniso(float NdV, float VdX, float VdY, float ax, float ay) { 
     return (2.0f * NdV) / (NdV + sqrtf_((a * a + b * b) + c * c));
 }
 
-RT_D V3 eval_microfacet_refraction(V3 bc, float anisotropic, float roughness, float eta, V3 V, V3 L, V3 H,
+RT_D V3 eval_microfacet_refraction(V3 bc, float ax, float ay, float eta, V3 V, V3 L, V3 H,
                                    float& pdf) {                            // :441-467
-    float ax, ay;
-    alphas(anisotropic, roughness, ax, ay);
     pdf = 0.0f;
     if (L.z >= 0.0f) return v3(0.0f, 0.0f, 0.0f);
     float LdH = dot(L, H), VdH = dot(V, H);
@@ -434,24 +468,28 @@ RT_D V3 eval_microfacet_refraction(V3 bc, float anisotropic, float roughness, fl
 // branch_pdf: the pdf includes the probability of sample_glass's branch, F for
 // reflection (1 under total internal reflection) and 1 - F for refraction
 // (REINA_RT_TRACE_FIX_DISNEY_MIX); the reference leaves it out.
-RT_D V3 eval_glass(const M3& tbn, V3 bc, float anisotropic, float roughness, float eta, V3 n, V3 wi, V3 wo,
-                   bool didRefract, bool bounded, bool branch_pdf, float& pdf) {   // :539-581
-    V3 h = didRefract ? normalize(add(wo, scale(wi, eta))) : normalize(add(wo, wi));
-    if (dot(h, n) < 0.0f) h = neg(h);
-    const V3 wiT = tmul(tbn, wi), hT = tmul(tbn, h);
+// terms, mp: the metal lobe's metal_terms(h) and pdf_metal for h = |wi + wo|,
+// which the reflection evaluates again in the reference.
+RT_D V3 eval_glass(const M3& tbn, V3 bc, float ax, float ay, float eta, V3 n, V3 wi, V3 wo, V3 h, const GgxTerms& terms,
+                   float mp, bool didRefract, bool branch_pdf, float& pdf) {   // :539-581
     if (didRefract) {
+        h = normalize(add(wo, scale(wi, eta)));
+        if (dot(h, n) < 0.0f) h = neg(h);
+        const V3 wiT = tmul(tbn, wi), hT = tmul(tbn, h);
         float tp;
-        V3 f = eval_microfacet_refraction(bc, anisotropic, roughness, eta, wiT, tmul(tbn, wo), hT, tp);
+        V3 f = eval_microfacet_refraction(bc, ax, ay, eta, wiT, tmul(tbn, wo), hT, tp);
         pdf = branch_pdf ? tp * (1.0f - reflectance(dot(wiT, hT), eta)) : tp;
         return f;
     }
-    pdf = pdf_metal(tbn, wi, wo, anisotropic, roughness, bounded);
+    pdf = mp;
     if (branch_pdf) {
+        if (dot(h, n) < 0.0f) h = neg(h);
+        const V3 wiT = tmul(tbn, wi), hT = tmul(tbn, h);
         const float c = dot(wiT, hT);
         const float s = sqrtf_(1.0f - c * c);
         pdf = pdf * ((eta * s > 1.0f) ? 1.0f : reflectance(c, eta));
     }
-    return eval_metal(tbn, bc, anisotropic, roughness, n, wi, wo, h, 0.0f, v3(1.0f, 1.0f, 1.0f), 1.0f, eta);
+    return metal_value(eval_fm(bc, h, wo, 0.0f, v3(1.0f, 1.0f, 1.0f), 1.0f, eta), terms);
 }
 
 RT_D V3 eval_sheen(V3 bc, V3 wo, V3 h, V3 n, V3 sheenTint) {               // :587-594
@@ -462,7 +500,7 @@ RT_D V3 eval_sheen(V3 bc, V3 wo, V3 h, V3 n, V3 sheenTint) {               // :5
     return scale(scale(cs, p), maxf_(dot(n, wo), 0.0f));
 }
 
-RT_D V3 sample_disney(const M3& tbn, float anisotropic, float roughness, float cg, float eta, float metallic,
+RT_D V3 sample_disney(const M3& tbn, const MaterialRec& mr, float cg, float eta, float metallic,
                       float clearcoat, float st, V3 n, V3 wi, bool& didRefract, bool& choseGlass,
                       uint32_t& rng) {                                      // :609-654
     float dW = (1.0f - st) * (1.0f - metallic);
@@ -474,14 +512,14 @@ RT_D V3 sample_disney(const M3& tbn, float anisotropic, float roughness, float c
     float r = rnd(rng) * cdf3;
     choseGlass = false;
     if (r < cdf0) return sample_diffuse(n, rng);
-    if (r < cdf1) return sample_metal(tbn, anisotropic, roughness, wi, rng);
+    if (r < cdf1) return sample_metal(tbn, mr.ax, mr.ay, wi, rng);
     if (r < cdf2) return sample_clearcoat(tbn, cg, wi, rng);
     choseGlass = true;
-    return sample_glass(tbn, wi, roughness, anisotropic, eta, rng, didRefract);
+    return sample_glass(tbn, wi, mr.ax, mr.ay, eta, rng, didRefract);
 }
 
-RT_D V3 eval_disney(const M3& tbn, V3 bc, V3 specularTint, V3 sheenTint, float anisotropic, float roughness,
-                    float subsurface, float cg, float eta, float metallic, float clearcoat, float st, float sheen,
+RT_D V3 eval_disney(const M3& tbn, const MaterialRec& mr, V3 bc, V3 specularTint, V3 sheenTint, float roughness,
+                    float subsurface, float eta, float metallic, float clearcoat, float st, float sheen,
                     bool didRefract, uint32_t fixes, V3 n, V3 wi, V3 wo, V3 h, float& pdf) { // :656-711
     // fixes: REINA_RT_TRACE_FIX_METAL_PDF (sampler density for GGX reflection),
     // REINA_RT_TRACE_FIX_DISNEY_MIX (clearcoat inside the normalised mixture,
@@ -492,23 +530,29 @@ RT_D V3 eval_disney(const M3& tbn, V3 bc, V3 specularTint, V3 sheenTint, float a
     float mW = metallic;
     float cW = 0.25f * clearcoat;
     float gW = (1.0f - metallic) * st;
-    float ws = (dW + mW) + gW;
-    if (mix) ws = ws + cW;
-    const float cN = mix ? cW / ws : cW;
+    float ws = mr.ws, dWn = mr.dWn, mWn = mr.mWn, gWn = mr.gWn, cN = cW;
+    if (mix) {
+        ws = ((dW + mW) + gW) + cW;
+        dWn = dW / ws;
+        mWn = mW / ws;
+        gWn = gW / ws;
+        cN = cW / ws;
+    }
     V3 fd = eval_diffuse(roughness, subsurface, bc, n, wi, wo, h);
     float dP = pdf_diffuse(wo, n);
     V3 fs = eval_sheen(bc, wo, h, n, sheenTint);
-    V3 fm = eval_metal(tbn, bc, anisotropic, roughness, n, wi, wo, h, mix ? 1.0f : st, specularTint, metallic, eta);
-    float mP = pdf_metal(tbn, wi, wo, anisotropic, roughness, bounded);
-    V3 fc = eval_clearcoat(tbn, wi, wo, cg, h);
-    float cP = pdf_clearcoat(tbn, wi, wo, h, cg);
+    const GgxTerms terms = metal_terms(tbn, mr.ax, mr.ay, n, wi, wo, h);
+    V3 fm = metal_value(eval_fm(bc, h, wo, mix ? 1.0f : st, specularTint, metallic, eta), terms);
+    float mP = pdf_metal(tbn, wi, wo, mr.ax, mr.ay, bounded);
+    V3 fc = eval_clearcoat(tbn, wi, wo, mr, h);
+    float cP = pdf_clearcoat(tbn, wi, wo, h, mr);
     float gP;
-    V3 fg = eval_glass(tbn, bc, anisotropic, roughness, eta, n, wi, wo, didRefract, bounded, mix, gP);
+    V3 fg = eval_glass(tbn, bc, mr.ax, mr.ay, eta, n, wi, wo, h, terms, mP, didRefract, mix, gP);
     pdf = (((dP * dW) / ws + (mP * mW) / ws) + cP * cN) + (gP * gW) / ws;
-    V3 r = scale(add(fd, scale(fs, sheen)), dW / ws);
-    r = add(r, scale(fm, mW / ws));
+    V3 r = scale(add(fd, scale(fs, sheen)), dWn);
+    r = add(r, scale(fm, mWn));
     r = add(r, scale(fc, cN));
-    r = add(r, scale(fg, gW / ws));
+    r = add(r, scale(fg, gWn));
     return r;
 }
 
@@ -545,23 +589,21 @@ RT_D float vndf_reflection_density(V3 wiT, V3 woT, float ax, float ay) {
     return (eval_dm(m, ax, ay) * smith_g(wiT, ax, ay)) / (4.0f * wiT.z);
 }
 
-RT_D void disney_density(const M3& tbn, float anisotropic, float roughness, float cg, float eta, float metallic,
+RT_D void disney_density(const M3& tbn, const MaterialRec& rec, float eta, float metallic,
                          float clearcoat, float st, V3 n, V3 wi, V3 wo, float& png, float& pg) {
     const float dW = (1.0f - st) * (1.0f - metallic);
     const float mW = metallic;
     const float cW = 0.25f * clearcoat;
     const float gW = (1.0f - metallic) * st;
     const float ws = ((dW + mW) + gW) + cW;
-    float ax, ay;
-    alphas(anisotropic, roughness, ax, ay);
+    const float ax = rec.ax, ay = rec.ay;
     const V3 wiT = tmul(tbn, wi), woT = tmul(tbn, wo);
     const float dP = pdf_diffuse(wo, n);
     const float mr = vndf_reflection_density(wiT, woT, ax, ay);
-    const float ag = (1.0f - cg) * 0.1f + cg * 0.001f;
     V3 hc = normalize(add(wiT, woT));
     if (hc.z < 0.0f) hc = neg(hc);
     const float ohc = fabsf(dot(woT, hc));
-    const float cP = ohc > 0.0f ? (eval_dc(ag, hc) * hc.z) / (4.0f * ohc) : 0.0f;
+    const float cP = ohc > 0.0f ? (eval_dc(rec, hc) * hc.z) / (4.0f * ohc) : 0.0f;
     float gr = 0.0f, gt = 0.0f;
     if (mr > 0.0f) {
         const V3 m = normalize(add(wiT, woT));
@@ -593,14 +635,15 @@ struct DisneyNee {
 };
 
 // g(w) of a light sample along w, and the sampler's density there (ptot).
-RT_D V3 disney_nee_weight(const DisneyNee& c, const ReinaInstanceProperties& p, uint32_t fixes, V3 w, float& ptot) {
+RT_D V3 disney_nee_weight(const DisneyNee& c, const ReinaInstanceProperties& p, const MaterialRec& mr, uint32_t fixes,
+                          V3 w, float& ptot) {
     const V3 h = normalize(add(w, c.wi));
     float pdf_ev;
-    const V3 f = eval_disney(c.tbn, c.albedo, ldv3(p.specularTint), ldv3(p.sheenTint), p.anisotropic, p.roughness,
-                             p.subsurface, p.clearcoatGloss, c.eta, p.metallic, p.clearcoat, p.specularTransmission,
+    const V3 f = eval_disney(c.tbn, mr, c.albedo, ldv3(p.specularTint), ldv3(p.sheenTint), p.roughness,
+                             p.subsurface, c.eta, p.metallic, p.clearcoat, p.specularTransmission,
                              p.sheen, false, fixes, c.wn, c.wi, w, h, pdf_ev);
     float png, pg;
-    disney_density(c.tbn, p.anisotropic, p.roughness, p.clearcoatGloss, c.eta, p.metallic, p.clearcoat,
+    disney_density(c.tbn, mr, c.eta, p.metallic, p.clearcoat,
                    p.specularTransmission, c.wn, c.wi, w, png, pg);
     ptot = png + pg;
     const float cx = maxf_(dot(c.wn, w), 0.0f);
@@ -620,15 +663,29 @@ RT_D V3 disney_nee_weight(const DisneyNee& c, const ReinaInstanceProperties& p, 
 // linear interpolations along x and one along y. Hardware filtering rounds its weights to a few
 // fraction bits, so texel-edge values of the reference are implementation
 // defined; this order is the library's definition.
+// n / 255 for a whole n in 0..255, correctly rounded: the quotient by the
+// rounded reciprocal, corrected by its exact remainder (equal to the division
+// for all 256 values, tests/test_gpu_shading_math.py), 3 operations instead of
+// the 14 of a division
+RT_D float over255(uint32_t n) {
+    const float x = (float)n, c = 1.0f / 255.0f, q = x * c;
+    return __builtin_fmaf(__builtin_fmaf(-255.0f, q, x), c, q);
+}
 RT_D float4 unorm8(uint32_t t) {
-    return make_float4((float)(t & 0xFFu) / 255.0f, (float)((t >> 8) & 0xFFu) / 255.0f,
-                       (float)((t >> 16) & 0xFFu) / 255.0f, (float)(t >> 24) / 255.0f);
+    return make_float4(over255(t & 0xFFu), over255((t >> 8) & 0xFFu), over255((t >> 16) & 0xFFu), over255(t >> 24));
 }
 
-// floor(x) mod n for a floored, finite x with |x| <= 2^30
+// floor(x) mod n for a floored, finite x with |x| <= 2^30; coordinates in
+// (or within one texture of) the unit square, which is where uv mod 1 and a
+// bump search's steps lie, take no integer division
 RT_D uint32_t repeat_index(float fx, uint32_t n) {
-    const int32_t m = (int32_t)fx % (int32_t)n;
-    return (uint32_t)(m < 0 ? m + (int32_t)n : m);
+    const int32_t i = (int32_t)fx, w = (int32_t)n;
+    int32_t m = i < 0 ? i + w : (i >= w ? i - w : i);
+    if ((uint32_t)m >= n) {
+        m = i % w;
+        m = m < 0 ? m + w : m;
+    }
+    return (uint32_t)m;
 }
 
 RT_D float4 tex_sample(const SceneView& sv, int32_t id, float u, float v) {
@@ -699,35 +756,66 @@ RT_D void skip_hit(Payload& pld, const HitInfo& hi, V3 D) {                // cl
     pld.skip = true;
 }
 
-// lambertian.rchit.glsl:11-78 (metal = false) and metal.rchit.glsl:7-70 (metal = true)
-RT_D void chs_lambert_metal(Payload& pld, const SceneView& sv, const HitInfo& hi, const ReinaInstanceProperties& p,
-                            V3 D, bool metal) {
-    if (p.cullBackface != 0u && !hi.frontFace) { skip_hit(pld, hi, D); return; }
-    float ux = hi.uvx - floorf(hi.uvx), uy = hi.uvy - floorf(hi.uvy);   // mod(uv, 1.0)
-    if (p.bumpMapTexID >= 0) bump_mapping(sv, p.bumpMapTexID, ux, uy, normalize(D), hi.tbn);
-    if (!metal && (ux < 0.0f || ux > 1.0f || uy < 0.0f || uy > 1.0f)) { skip_hit(pld, hi, D); return; }
-    V3 wn = hi.worldNormal;
-    if (p.normalMapTexID >= 0) wn = normal_map(sv, p.normalMapTexID, ux, uy, hi.tbn);
-    pld.color = ldv3(p.albedo);
-    if (p.textureID >= 0) {
-        const float4 tc = tex_sample(sv, p.textureID, ux, uy);
-        if (tc.w < 0.999f && rnd(pld.rng) > tc.w) { skip_hit(pld, hi, D); return; }   // transparency
-        pld.color = mul(pld.color, v3(tc.x, tc.y, tc.z));
+// What the four hit shaders begin with: back-face culling, bump mapping, the
+// uv range test, normal and albedo maps and the alpha test, in the order in
+// which each shader draws random numbers (one, for the alpha test). One copy
+// of the texture code for all of them: four made the shading kernels' code
+// larger than the instruction cache. Returns false for a skipped hit.
+struct Surface {
+    V3 albedo, wn;
+    M3 tbn;      // set for Disney surfaces and where a normal or bump map is present
+};
+RT_D bool hit_surface(Payload& pld, const SceneView& sv, const HitInfo& hi, const ReinaInstanceProperties& p,
+                      const InstanceRec RT_GLOBAL& in, const float4 RT_GLOBAL* rec, float f0, uint32_t prim,
+                      uint32_t material, V3 D, Surface& s) {
+    if (material != 2u && p.cullBackface != 0u && !hi.frontFace) { skip_hit(pld, hi, D); return false; }
+    s.wn = hi.worldNormal;
+    s.albedo = ldv3(p.albedo);
+    const bool mapped = p.normalMapTexID >= 0 || p.bumpMapTexID >= 0;
+    if (material == 3u || mapped) s.tbn = hit_tbn(in, rec, f0, hi);
+    if (mapped || p.textureID >= 0) {
+        float ux, uy;
+        hit_uv(sv, p, prim, hi, ux, uy);
+        ux = ux - floorf(ux);   // mod(uv, 1.0): in [0, 1], so the range test needs a bump map to fail
+        uy = uy - floorf(uy);
+        if (p.bumpMapTexID >= 0) {
+            bump_mapping(sv, p.bumpMapTexID, ux, uy, normalize(D), s.tbn);
+            if ((material == 0u || material == 3u) && (ux < 0.0f || ux > 1.0f || uy < 0.0f || uy > 1.0f)) {
+                skip_hit(pld, hi, D);
+                return false;
+            }
+        }
+        if (p.normalMapTexID >= 0) s.wn = normal_map(sv, p.normalMapTexID, ux, uy, s.tbn);
+        if (p.textureID >= 0) {
+            const float4 tc = tex_sample(sv, p.textureID, ux, uy);
+            if (material != 2u && tc.w < 0.999f && rnd(pld.rng) > tc.w) {   // transparency
+                skip_hit(pld, hi, D);
+                return false;
+            }
+            s.albedo = mul(s.albedo, v3(tc.x, tc.y, tc.z));
+        }
     }
-    pld.albedo = pld.color;
-    pld.surfaceNormal = wn;
+    return true;
+}
+
+// lambertian.rchit.glsl:11-78 (metal = false) and metal.rchit.glsl:7-70 (metal = true), after hit_surface
+RT_D void chs_lambert_metal(Payload& pld, const HitInfo& hi, const ReinaInstanceProperties& p, const Surface& s, V3 D,
+                            bool metal) {
+    pld.color = s.albedo;
+    pld.albedo = s.albedo;
+    pld.surfaceNormal = s.wn;
     pld.emission = ldv3(p.emission);
     pld.rayOrigin = offset_along(hi.worldPosition, hi.worldNormalGeometry);
-    if (!metal) pld.rayDirection = diffuse_reflection(wn, pld.rng);
-    else pld.rayDirection = fuzzy_reflection(D, wn, p.roughness, pld.rng);
+    if (!metal) pld.rayDirection = diffuse_reflection(s.wn, pld.rng);
+    else pld.rayDirection = fuzzy_reflection(D, s.wn, p.roughness, pld.rng);
     pld.rayHitSky = false;
     pld.skip = false;
     pld.insideDielectric = false;
     pld.accumulatedDistance = 0.0f;
 }
 
-// dielectric.rchit.glsl:40-113
-RT_D void chs_dielectric(Payload& pld, const SceneView& sv, const HitInfo& hi, const ReinaInstanceProperties& p, V3 O,
+// dielectric.rchit.glsl:40-113, after hit_surface
+RT_D void chs_dielectric(Payload& pld, const HitInfo& hi, const ReinaInstanceProperties& p, const Surface& s, V3 O,
                          V3 D) {
     float ri = hi.frontFace ? 1.0f / p.ior : p.ior;
     V3 unitDir = normalize(D);
@@ -736,68 +824,47 @@ RT_D void chs_dielectric(Payload& pld, const SceneView& sv, const HitInfo& hi, c
     bool cannot = ri * sinTheta > 1.0f;
     float refl = reflectance(cosTheta, ri);
     bool prevInside = pld.insideDielectric;
-    float ux = hi.uvx - floorf(hi.uvx), uy = hi.uvy - floorf(hi.uvy);   // mod(uv, 1.0)
-    if (p.bumpMapTexID >= 0) bump_mapping(sv, p.bumpMapTexID, ux, uy, normalize(D), hi.tbn);
-    V3 albedo = ldv3(p.albedo);
-    if (p.textureID >= 0) {
-        const float4 tc = tex_sample(sv, p.textureID, ux, uy);
-        albedo = mul(albedo, v3(tc.x, tc.y, tc.z));
-    }
-    V3 wn = hi.worldNormal;
-    if (p.normalMapTexID >= 0) wn = normal_map(sv, p.normalMapTexID, ux, uy, hi.tbn);
     if (cannot || refl > rnd(pld.rng)) {
-        pld.rayDirection = fuzzy_reflection(unitDir, wn, p.roughness, pld.rng);
+        pld.rayDirection = fuzzy_reflection(unitDir, s.wn, p.roughness, pld.rng);
         pld.color = v3(1.0f, 1.0f, 1.0f);
         pld.rayOrigin = offset_along(hi.worldPosition, hi.worldNormalGeometry);
     } else {
         pld.insideDielectric = hi.frontFace;
-        pld.rayDirection = add(refract(unitDir, wn, ri), scale(random_unit_vec(pld.rng), p.roughness));
-        pld.color = albedo;
+        pld.rayDirection = add(refract(unitDir, s.wn, ri), scale(random_unit_vec(pld.rng), p.roughness));
+        pld.color = s.albedo;
         pld.rayOrigin = offset_dielectric(hi.worldPosition, hi.worldNormalGeometry, unitDir);
     }
     pld.accumulatedDistance = pld.accumulatedDistance + (prevInside ? length(sub(hi.worldPosition, O)) : 0.0f);
     if (prevInside && !pld.insideDielectric) {
         float e = expf_(-p.absorption * pld.accumulatedDistance);
-        pld.color = mul(v3(e, e, e), albedo);
+        pld.color = mul(v3(e, e, e), s.albedo);
         pld.accumulatedDistance = 0.0f;
     }
     pld.albedo = pld.color;
-    pld.surfaceNormal = wn;
+    pld.surfaceNormal = s.wn;
     pld.emission = ldv3(p.emission);
     pld.rayHitSky = false;
     pld.skip = false;
 }
 
-// disney.rchit.glsl:36-198
+// disney.rchit.glsl:36-198, after hit_surface
 // fixes: the REINA_RT_TRACE_FIX_* bits of the trace (eval_disney reads two)
-RT_D void chs_disney(Payload& pld, const SceneView& sv, const HitInfo& hi, const ReinaInstanceProperties& p, V3 O,
-                     V3 D, uint32_t fixes, DisneyNee* dn = nullptr) {
-    if (p.cullBackface != 0u && !hi.frontFace) { skip_hit(pld, hi, D); return; }
-    float ux = hi.uvx - floorf(hi.uvx), uy = hi.uvy - floorf(hi.uvy);   // mod(uv, 1.0)
-    if (p.bumpMapTexID >= 0) bump_mapping(sv, p.bumpMapTexID, ux, uy, normalize(D), hi.tbn);
-    if (ux < 0.0f || ux > 1.0f || uy < 0.0f || uy > 1.0f) { skip_hit(pld, hi, D); return; }
-    V3 wn = hi.worldNormal;
-    if (p.normalMapTexID >= 0) wn = normal_map(sv, p.normalMapTexID, ux, uy, hi.tbn);
-    V3 albedo = ldv3(p.albedo);
-    if (p.textureID >= 0) {
-        const float4 tc = tex_sample(sv, p.textureID, ux, uy);
-        if (tc.w < 0.999f && rnd(pld.rng) > tc.w) { skip_hit(pld, hi, D); return; }   // transparency
-        albedo = mul(albedo, v3(tc.x, tc.y, tc.z));
-    }
+RT_D void chs_disney(Payload& pld, const HitInfo& hi, const ReinaInstanceProperties& p, const MaterialRec& mr,
+                     const Surface& s, V3 O, V3 D, uint32_t fixes, DisneyNee* dn = nullptr) {
     float eta = hi.frontFace ? 1.0f / p.ior : p.ior;
     bool didRefract = false, choseGlass = false;
     V3 wi = neg(D);
-    V3 rayDir = sample_disney(hi.tbn, p.anisotropic, p.roughness, p.clearcoatGloss, eta, p.metallic, p.clearcoat,
-                              p.specularTransmission, wn, wi, didRefract, choseGlass, pld.rng);
+    V3 rayDir = sample_disney(s.tbn, mr, p.clearcoatGloss, eta, p.metallic, p.clearcoat,
+                              p.specularTransmission, s.wn, wi, didRefract, choseGlass, pld.rng);
     V3 h = normalize(add(rayDir, wi));
     float pdf;
-    V3 f = eval_disney(hi.tbn, albedo, ldv3(p.specularTint), ldv3(p.sheenTint), p.anisotropic, p.roughness,
-                       p.subsurface, p.clearcoatGloss, eta, p.metallic, p.clearcoat, p.specularTransmission, p.sheen,
-                       didRefract, fixes, wn, wi, rayDir, h, pdf);
-    float cosThetaI = maxf_(dot(wn, rayDir), 0.0f);
+    V3 f = eval_disney(s.tbn, mr, s.albedo, ldv3(p.specularTint), ldv3(p.sheenTint), p.roughness,
+                       p.subsurface, eta, p.metallic, p.clearcoat, p.specularTransmission, p.sheen,
+                       didRefract, fixes, s.wn, wi, rayDir, h, pdf);
+    float cosThetaI = maxf_(dot(s.wn, rayDir), 0.0f);
     pld.color = divs(scale(f, cosThetaI), pdf);
-    pld.albedo = albedo;
-    pld.surfaceNormal = wn;
+    pld.albedo = s.albedo;
+    pld.surfaceNormal = s.wn;
     pld.emission = ldv3(p.emission);
     pld.rayOrigin = offset_dielectric(hi.worldPosition, hi.worldNormalGeometry, rayDir);
     pld.rayDirection = rayDir;
@@ -809,16 +876,16 @@ RT_D void chs_disney(Payload& pld, const SceneView& sv, const HitInfo& hi, const
     else
         pld.accumulatedDistance = 0.0f;
     if (dn) {
-        dn->tbn = hi.tbn;
-        dn->albedo = albedo;
-        dn->wn = wn;
+        dn->tbn = s.tbn;
+        dn->albedo = s.albedo;
+        dn->wn = s.wn;
         dn->wi = wi;
         dn->pos = hi.worldPosition;
         dn->ng = hi.worldNormalGeometry;
         dn->eta = eta;
         float png, pg;
-        disney_density(hi.tbn, p.anisotropic, p.roughness, p.clearcoatGloss, eta, p.metallic, p.clearcoat,
-                       p.specularTransmission, wn, wi, rayDir, png, pg);
+        disney_density(s.tbn, mr, eta, p.metallic, p.clearcoat,
+                       p.specularTransmission, s.wn, wi, rayDir, png, pg);
         dn->p_bsdf = png + pg;
     }
 }
@@ -829,6 +896,7 @@ struct Camera {
     float invProj[16];
     float focusDist, defocus;
     float W, H;
+    V3 right, up;   // unit camera axes, normalize(invView[0..2]) and normalize(invView[4..6])
 };
 
 RT_D void m4mul(const float* m, float x, float y, float z, float w, float* o) {
@@ -868,9 +936,7 @@ RT_D void starting_ray(const Camera& cam, float px, float py, uint32_t& rng, V3&
     } while (fabsf(hy) > sqrt3 * 0.5f || (sqrt3 * fabsf(hx) + fabsf(hy)) > sqrt3);
     if (lens_advances) rng = hr;
     float lx = hx * cam.defocus, ly = hy * cam.defocus;
-    V3 right = normalize(v3(cam.invView[0], cam.invView[1], cam.invView[2]));
-    V3 up = normalize(v3(cam.invView[4], cam.invView[5], cam.invView[6]));
-    V3 no = add(origin, add(scale(right, lx), scale(up, ly)));
+    V3 no = add(origin, add(scale(cam.right, lx), scale(cam.up, ly)));
     o = no;
     d = normalize(sub(focal, no));
 }

@@ -55,9 +55,10 @@ RT_D uint32_t cdf_pick(uint32_t lo, uint32_t hi, float u, F cdf) {
 
 // World-space vertices of triangle `prim` of instance `in`, bit-identical to
 // the flattened triangles of the BVH (((c0 x + c1 y) + c2 z) + c3).
-RT_D void world_triangle(const SceneView& sv, const InstanceRec& in, const ReinaInstanceProperties& p, uint32_t prim,
+RT_D void world_triangle(const SceneView& sv, const InstanceRec RT_GLOBAL& in, const ReinaInstanceProperties& p, uint32_t prim,
                          V3& w0, V3& w1, V3& w2) {
-    const V3 c0 = ldv3(in.c0), c1 = ldv3(in.c1), c2 = ldv3(in.c2), c3 = ldv3(in.c3);
+    const V3 c0 = v3(in.c0[0], in.c0[1], in.c0[2]), c1 = v3(in.c1[0], in.c1[1], in.c1[2]);
+    const V3 c2 = v3(in.c2[0], in.c2[1], in.c2[2]), c3 = v3(in.c3[0], in.c3[1], in.c3[2]);
     V3 w[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -100,6 +101,7 @@ RT_D ShadeResult shade_ray(const SceneView& sv, const TraceParams& P, const Path
     bool lambert_hit = false, disney_hit = false, emissive_mis = false;
     DisneyNee dn;
     const ReinaInstanceProperties* hp = nullptr;
+    const MaterialRec RT_GLOBAL* hm = nullptr;
     V3 nee_n = r.no, nee_albedo = r.no;
     float emis_w = 1.0f;
     uint4 s0 = S.st0[pp];
@@ -121,21 +123,28 @@ RT_D ShadeResult shade_ray(const SceneView& sv, const TraceParams& P, const Path
         pld.rayHitSky = true;
         pld.skip = false;
     } else {
-        const float4* rec = sv.srec + (size_t)kShadeRecF4 * prim;
-        const uint32_t ii = __float_as_uint(rec[0].w), pm = __float_as_uint(rec[1].w);
-        const InstanceRec in = sv.inst[ii];
-        const ReinaInstanceProperties& pr = sv.props[__float_as_uint(rec[2].w)];
-        HitInfo hi = hit_info(sv, in, pr, rec, pm, hh.z, hh.w, D, (P.fixes & REINA_RT_TRACE_FIX_NORMALS) != 0u);
-        switch (in.material) {
-            case 0: chs_lambert_metal(pld, sv, hi, pr, D, false); break;
-            case 1: chs_lambert_metal(pld, sv, hi, pr, D, true); break;
-            case 2: chs_dielectric(pld, sv, hi, pr, O, D); break;
-            default: chs_disney(pld, sv, hi, pr, O, D, P.fixes, nee ? &dn : nullptr); break;
+        const float4 RT_GLOBAL* rec = sv.srec + (size_t)kShadeRecF4 * prim;
+        const float4 rq[4] = {rec[0], rec[1], rec[2], rec[3]};
+        const uint32_t ii = __float_as_uint(rq[0].w), pm = __float_as_uint(rq[1].w), pi = __float_as_uint(rq[2].w);
+        const InstanceRec RT_GLOBAL& in = sv.inst[ii];
+        const ReinaInstanceProperties& pr = sv.props[pi];
+        const uint32_t material = in.material;
+        const HitInfo hi = hit_info(in, pr.interpNormals != 0, rec, rq, hh.z, hh.w, D,
+                                    (P.fixes & REINA_RT_TRACE_FIX_NORMALS) != 0u);
+        Surface sf;
+        if (hit_surface(pld, sv, hi, pr, in, rec, rq[3].w, pm, material, D, sf)) {
+            switch (material) {
+                case 0: chs_lambert_metal(pld, hi, pr, sf, D, false); break;
+                case 1: chs_lambert_metal(pld, hi, pr, sf, D, true); break;
+                case 2: chs_dielectric(pld, hi, pr, sf, O, D); break;
+                default: chs_disney(pld, hi, pr, sv.mats[pi], sf, O, D, P.fixes, nee ? &dn : nullptr); break;
+            }
         }
         if (nee && !pld.skip) {
-            lambert_hit = in.material == 0u;
-            disney_hit = in.material == 3u;
+            lambert_hit = material == 0u;
+            disney_hit = material == 3u;
             hp = &pr;
+            hm = &sv.mats[pi];
             nee_n = pld.surfaceNormal;     // the shading normal (normal-mapped) and
             nee_albedo = pld.albedo;       // textured colour of the Lambertian BSDF
             // an emitter reached by the continuation of a Lambertian bounce: MIS weight
@@ -172,7 +181,7 @@ RT_D ShadeResult shade_ray(const SceneView& sv, const TraceParams& P, const Path
                 const EmissiveInst ei = sv.emi[k];
                 const uint32_t t = cdf_pick(ei.cdf_base, ei.cdf_base + ei.ntri - 1u, u2,
                                             [&](uint32_t i) { return sv.tri_cdf[i]; }) - ei.cdf_base;
-                const InstanceRec li = sv.inst[ei.inst];
+                const InstanceRec RT_GLOBAL& li = sv.inst[ei.inst];
                 const ReinaInstanceProperties& lp = sv.props[li.props_id];
                 V3 w0, w1, w2;
                 world_triangle(sv, li, lp, t, w0, w1, w2);
@@ -208,7 +217,7 @@ RT_D ShadeResult shade_ray(const SceneView& sv, const TraceParams& P, const Path
                     const float pl = light_pdf(ei.pdf_area, dist, ng, w, lp.cullBackface != 0u);
                     if (pl > 0.0f && dist > 0.001f) {
                         float pt;
-                        const V3 g = disney_nee_weight(dn, *hp, P.fixes, w, pt);
+                        const V3 g = disney_nee_weight(dn, *hp, *hm, P.fixes, w, pt);
                         if (g.x > 0.0f || g.y > 0.0f || g.z > 0.0f) {
                             const float wn = power_heuristic(pl, pt);
                             r.scontrib = mul(scale(mul(ldv3(lp.emission), g), wn / pl), thr);

@@ -1,0 +1,46 @@
+"""The shading kernels' shortcuts against what they stand for: whole numbers
+over 255, texel indices without an integer division, the tangent frame left
+out where no surface reads it."""
+import numpy as np
+import pytest
+
+import oracle
+import reina_rt
+from reina_rt import scenes
+from reina_rt.scene import make_desc
+
+
+def test_over_255_is_the_rounded_quotient():
+    """n * c corrected by its exact remainder equals n / 255 for every texel
+    value (products of two float32 are exact in float64, so each fused
+    multiply-add is one float64 expression rounded once)."""
+    n = np.arange(256, dtype=np.float32)
+    c = np.float32(1.0) / np.float32(255.0)
+    q = n * c
+    r = (np.float64(-255.0) * q.astype(np.float64) + n).astype(np.float32)
+    got = (r.astype(np.float64) * np.float64(c) + q).astype(np.float32)
+    assert np.array_equal(got, n / np.float32(255.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,h", [(1, 1), (3, 5), (257, 2)])
+def test_texture_sizes_equal_oracle(cuda, w, h):
+    """Odd texture sizes on every map: the bump search at grazing angles walks
+    many textures away, past what one wrap brings back. Lambertian walls
+    without maps and mapped ones lie in one frame, so waves mix surfaces with
+    and without a tangent frame."""
+    torch = cuda
+    sc, _ = scenes.textured_cornell()
+    arrays = sc.build_arrays()
+    rng = np.random.default_rng(w * 100 + h)
+    arrays["textures"] = [rng.integers(0, 256, (h, w, 4), dtype=np.uint8) for _ in arrays["textures"]]
+    W, H = 40, 36
+    pc = scenes.cornell_push(W, H, spp=3, max_bounces=6)
+    dev = reina_rt.DeviceScene(arrays)
+    img = torch.zeros((H, W, 4), device="cuda")
+    dev.trace(pc, img.data_ptr(), W, H)
+    torch.cuda.synchronize()
+    ref, _ = oracle.OracleScene(arrays, make_desc).render(pc, W, H, use_bvh=False)
+    got = img.cpu().numpy()
+    assert ((got.view(np.uint32) == ref.view(np.uint32)) | (np.isnan(got) & np.isnan(ref))).all()
+    dev.close()
