@@ -183,6 +183,8 @@ __global__ void k_debug_math(int fn, const float* in, const float* in2, float* o
         case 4: r = sqrtf_(x); break;
         case 5: r = powf_(x, in2[i]); break;
         case 6: r = exp2f_(x); break;
+        case 7: r = inv_(x); break;
+        case 8: r = inv_sqrt_(x); break;
         default: r = __builtin_nanf("");
     }
     out[i] = r;

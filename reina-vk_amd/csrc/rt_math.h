@@ -139,37 +139,45 @@ RT_D float pow5_(float x) { float x2 = x * x; return (x2 * x2) * x; }
 // results equal the compiler's for every float of those ranges (2^-100 to
 // 2^126 for the root, 2^-124 to 2^125 for the inverse: all 1.9 and 2.1
 // billion inputs compared on the device, tests/test_gpu_shading_math.py).
-// The rest (zero, subnormal, infinite, NaN, negative) takes the compiler's.
+// For the rest (zero, subnormal, infinite, NaN, negative) the wave branches to
+// the compiler's form: a scalar branch on the ballot, which costs the common
+// case no exec-mask work.
 RT_HD float sqrtf_(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    if (__builtin_expect(__float_as_uint(x) - 0x0D800000u < 0x7E800000u - 0x0D800000u, 1)) {
-        const float y = __builtin_amdgcn_rsqf(x), g = x * y, h = 0.5f * y;
-        return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
-    }
-#endif
+    const float y = __builtin_amdgcn_rsqf(x), g = x * y, h = 0.5f * y;
+    float s = __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+    const bool rare = __float_as_uint(x) - 0x0D800000u >= 0x7E800000u - 0x0D800000u;
+    if (__builtin_expect(__ballot(rare) != 0ull, 0)) s = rare ? __builtin_sqrtf(x) : s;
+    return s;
+#else
     return __builtin_sqrtf(x);
+#endif
 }
 // 1 / x
 RT_HD float inv_(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    if (__builtin_expect((__float_as_uint(x) & 0x7FFFFFFFu) - 0x01800000u < 0x7E000000u - 0x01800000u, 1)) {
-        const float y = __builtin_amdgcn_rcpf(x);
-        return __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
-    }
-#endif
+    const float y = __builtin_amdgcn_rcpf(x);
+    float r = __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
+    const bool rare = (__float_as_uint(x) & 0x7FFFFFFFu) - 0x01800000u >= 0x7E000000u - 0x01800000u;
+    if (__builtin_expect(__ballot(rare) != 0ull, 0)) r = rare ? 1.0f / x : r;
+    return r;
+#else
     return 1.0f / x;
+#endif
 }
 // 1 / sqrt(x), each rounded
 RT_HD float inv_sqrt_(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    if (__builtin_expect(__float_as_uint(x) - 0x0D800000u < 0x7E800000u - 0x0D800000u, 1)) {
-        const float y = __builtin_amdgcn_rsqf(x), g = x * y, h = 0.5f * y;
-        const float s = __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
-        const float z = __builtin_amdgcn_rcpf(s);
-        return __builtin_fmaf(__builtin_fmaf(-s, z, 1.0f), z, z);
-    }
-#endif
+    const float y = __builtin_amdgcn_rsqf(x), g = x * y, h = 0.5f * y;
+    const float s = __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+    const float z = __builtin_amdgcn_rcpf(s);
+    float r = __builtin_fmaf(__builtin_fmaf(-s, z, 1.0f), z, z);
+    const bool rare = __float_as_uint(x) - 0x0D800000u >= 0x7E800000u - 0x0D800000u;
+    if (__builtin_expect(__ballot(rare) != 0ull, 0)) r = rare ? 1.0f / __builtin_sqrtf(x) : r;
+    return r;
+#else
     return 1.0f / __builtin_sqrtf(x);
+#endif
 }
 
 RT_D int32_t f2i_(float x) {

@@ -234,7 +234,7 @@ RT_D V3 sample_ggx_vndf(V3 V, float ax, float ay, uint32_t& rng) {         // :9
     float r2 = rnd(rng);
     V3 Vh = normalize(v3(ax * V.x, ay * V.y, V.z));
     float lensq = Vh.x * Vh.x + Vh.y * Vh.y;
-    V3 T1 = lensq > 0.0f ? scale(v3(-Vh.y, Vh.x, 0.0f), 1.0f / sqrtf_(lensq)) : v3(1.0f, 0.0f, 0.0f);
+    V3 T1 = lensq > 0.0f ? scale(v3(-Vh.y, Vh.x, 0.0f), inv_sqrt_(lensq)) : v3(1.0f, 0.0f, 0.0f);
     V3 T2 = cross(Vh, T1);
     float r = sqrtf_(r1);
     float phi = (2.0f * kPi) * r2;
@@ -251,7 +251,7 @@ RT_D V3 sample_ggx_vndf(V3 V, float ax, float ay, uint32_t& rng) {         // :9
 
 RT_D float d_ggx_aniso(V3 m, float ax, float ay) {                          // :42-48
     float NoM = maxf_(m.z, 0.0f);
-    float inv = 1.0f / (((m.x / ax) * (m.x / ax) + (m.y / ay) * (m.y / ay)) + NoM * NoM);
+    float inv = inv_(((m.x / ax) * (m.x / ax) + (m.y / ay) * (m.y / ay)) + NoM * NoM);
     return (inv * inv) / ((kPi * ax) * ay);
 }
 
@@ -296,7 +296,7 @@ RT_D V3 eval_diffuse(float roughness, float subsurface, V3 bc, V3 n, V3 wi, V3 w
     float fss90 = (roughness * hw) * hw;
     float fssIn = 1.0f + (fss90 - 1.0f) * pow5_(1.0f - maxf_(dot(n, wi), 0.0f));
     float fssOut = 1.0f + (fss90 - 1.0f) * pow5_(1.0f - maxf_(dot(n, wo), 0.0f));
-    float third = 1.0f / (maxf_(dot(n, wi), 0.0f) + maxf_(dot(n, wo), 0.0f)) - 0.5f;
+    float third = inv_(maxf_(dot(n, wi), 0.0f) + maxf_(dot(n, wo), 0.0f)) - 0.5f;
     V3 subs = scale(k, (fssIn * fssOut) * third + 0.5f);
     return mix(base, subs, subsurface);
 }
@@ -336,12 +336,12 @@ RT_D V3 eval_fm(V3 bc, V3 h, V3 wo, float specular, V3 specularTint, float metal
 RT_D float eval_dm(V3 hl, float ax, float ay) {                             // :224-229
     float constant = (kPi * ax) * ay;
     float q = (pow2_(hl.x) / pow2_(ax) + pow2_(hl.y) / pow2_(ay)) + pow2_(hl.z);
-    return 1.0f / (constant * pow2_(q));
+    return inv_(constant * pow2_(q));
 }
 
 RT_D float smith_g(V3 wl, float ax, float ay) {                             // :231-239
     float st = sqrtf_(1.0f + (pow2_(wl.x * ax) + pow2_(wl.y * ay)) / pow2_(wl.z));
-    return 1.0f / (1.0f + (st - 1.0f) / 2.0f);
+    return inv_(1.0f + (st - 1.0f) / 2.0f);
 }
 
 RT_HD void alphas(float anisotropic, float roughness, float& ax, float& ay) {
@@ -817,7 +817,7 @@ RT_D void chs_lambert_metal(Payload& pld, const HitInfo& hi, const ReinaInstance
 // dielectric.rchit.glsl:40-113, after hit_surface
 RT_D void chs_dielectric(Payload& pld, const HitInfo& hi, const ReinaInstanceProperties& p, const Surface& s, V3 O,
                          V3 D) {
-    float ri = hi.frontFace ? 1.0f / p.ior : p.ior;
+    float ri = hi.frontFace ? inv_(p.ior) : p.ior;
     V3 unitDir = normalize(D);
     float cosTheta = minf_(dot(neg(unitDir), hi.worldNormal), 1.0f);
     float sinTheta = sqrtf_(1.0f - cosTheta * cosTheta);
@@ -851,7 +851,7 @@ RT_D void chs_dielectric(Payload& pld, const HitInfo& hi, const ReinaInstancePro
 // fixes: the REINA_RT_TRACE_FIX_* bits of the trace (eval_disney reads two)
 RT_D void chs_disney(Payload& pld, const HitInfo& hi, const ReinaInstanceProperties& p, const MaterialRec& mr,
                      const Surface& s, V3 O, V3 D, uint32_t fixes, DisneyNee* dn = nullptr) {
-    float eta = hi.frontFace ? 1.0f / p.ior : p.ior;
+    float eta = hi.frontFace ? inv_(p.ior) : p.ior;
     bool didRefract = false, choseGlass = false;
     V3 wi = neg(D);
     V3 rayDir = sample_disney(s.tbn, mr, p.clearcoatGloss, eta, p.metallic, p.clearcoat,

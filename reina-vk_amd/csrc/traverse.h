@@ -67,9 +67,9 @@ RT_D void tray_init(TRay& r, float4 a, float4 b) {
     r.kx = kx; r.ky = ky; r.kz = kz;
     r.Sx = comp3(r.dx, r.dy, r.dz, kx) / dkz;
     r.Sy = comp3(r.dx, r.dy, r.dz, ky) / dkz;
-    r.Sz = 1.0f / dkz;
     // A zero component gives an infinite inverse (see node_hits).
-    r.ix = 1.0f / r.dx; r.iy = 1.0f / r.dy; r.iz = 1.0f / r.dz;
+    r.ix = inv_(r.dx); r.iy = inv_(r.dy); r.iz = inv_(r.dz);
+    r.Sz = comp3(r.ix, r.iy, r.iz, kz);
     if constexpr (H16) {
         auto normal16 = [](float v) { const float m = fabsf(v); return m >= 6.103515625e-05f && m <= 65504.0f; };
         if (normal16(r.ix) && normal16(r.iy) && normal16(r.iz)) {
@@ -116,7 +116,7 @@ RT_D bool wtest(const TRay& r, float4 p0, float4 p1, float4 p2, float tbest, flo
     if (det == 0.0f) return false;
     float Az = r.Sz * Akz, Bz = r.Sz * Bkz, Cz = r.Sz * Ckz;
     float T = (U * Az + V * Bz) + W * Cz;
-    float rcp = 1.0f / det;
+    float rcp = inv_(det);
     float t = T * rcp;
     if (!(t >= r.tmin && t <= tbest)) return false;
     to = t;

@@ -1,4 +1,5 @@
-"""The shading kernels' shortcuts against what they stand for: whole numbers
+"""The shading kernels' shortcuts against what they stand for: roots and
+inverses, whole numbers
 over 255, texel indices without an integer division, the tangent frame left
 out where no surface reads it."""
 import numpy as np
@@ -44,3 +45,28 @@ def test_texture_sizes_equal_oracle(cuda, w, h):
     got = img.cpu().numpy()
     assert ((got.view(np.uint32) == ref.view(np.uint32)) | (np.isnan(got) & np.isnan(ref))).all()
     dev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fn", [4, 7, 8], ids=["sqrt", "inverse", "inverse_sqrt"])
+def test_root_and_inverse_are_correctly_rounded(cuda, fn):
+    """sqrt, 1 / x and 1 / sqrt(x) against IEEE arithmetic on the host: every
+    mantissa of two neighbouring binades, every exponent, and the inputs
+    around the ends of the short forms' ranges."""
+    torch = cuda
+    man = np.arange(1 << 24, dtype=np.uint32) + np.uint32(0x3F800000)          # [1, 4)
+    exps = ((np.arange(256, dtype=np.uint32) << 23)[:, None] |
+            np.array([0, 1, 2, 0x2AAAAA, 0x3FFFFF, 0x400000, 0x7FFFFE, 0x7FFFFF], np.uint32)[None]).reshape(-1)
+    edge = (np.array([0x0D800000, 0x7E800000, 0x01800000, 0x7E000000], np.uint32)[:, None] +
+            np.arange(-8, 9).astype(np.uint32)[None]).reshape(-1)
+    bits = np.concatenate([man, exps, edge, exps | np.uint32(0x80000000), edge | np.uint32(0x80000000)])
+    x = bits.view(np.float32)
+    with np.errstate(all="ignore"):
+        ref = {4: np.sqrt(x), 7: np.float32(1.0) / x, 8: np.float32(1.0) / np.sqrt(x)}[fn]
+    t = torch.from_numpy(x.copy()).cuda()
+    out = torch.zeros_like(t)
+    reina_rt.debug_math(fn, t.data_ptr(), None, out.data_ptr(), len(x))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    same = (got.view(np.uint32) == ref.view(np.uint32)) | (np.isnan(got) & np.isnan(ref))
+    assert same.all(), [hex(b) for b in bits[~same][:8]]
