@@ -695,6 +695,21 @@ int reina_rt_set_trace_options(ReinaScene* s, uint32_t options) {
     return REINA_RT_OK;
 }
 
+// Batches of up to 2^18 rays take k_trace_once: every wave is resident at
+// once (4 per SIMD), so nothing is gained from a queue, whose launch needs its
+// counters cleared first and keeps a wave to claims of 128 rays. The rays are
+// spread over about 2,048 waves, two per SIMD: fewer lanes per wave then
+// diverge less. Per query, queue / once (bounce rays, us): icosphere 1,000
+// rays 72 / 48, 16,000 94 / 66, 65,536 110 / 76, 150,000 131 / 98, 300,000 137
+// / 138, 600,000 212 / 222; Cornell box 1,000 camera rays 30 / 13; 8-bit nodes,
+// 100,000 triangles: 65,536 89 / 59, 300,000 109 / 111.
+static constexpr uint32_t kOnceRays = 1u << 18;
+static uint32_t once_lanes_log2(uint32_t n) {
+    uint32_t l = 2;
+    while (l < 6u && (n >> l) > 2048u) ++l;
+    return l;
+}
+
 int reina_rt_intersect(ReinaScene* s, const ReinaRay* rays, ReinaHit* hits, uint32_t n, uint32_t* counters,
                        void* stream) {
     if (!s || (n && (!rays || !hits))) return fail(REINA_RT_ERR_INVALID_ARG, "null argument");
@@ -705,6 +720,11 @@ int reina_rt_intersect(ReinaScene* s, const ReinaRay* rays, ReinaHit* hits, uint
     if (n == 0) return REINA_RT_OK;
     const bool h16 = (s->options & REINA_RT_TRACE_F16_INV) != 0;
     if (h16 && s->sv.qnodes) return fail(REINA_RT_ERR_UNSUPPORTED, "FP16 inverse directions need FP32 nodes");
+    if (n <= kOnceRays) {
+        HIP_TRY(launch_trace_once(s->sv, (const float4*)rays, (float4*)hits, n, counters, h16, s->tune.stack_depth,
+                                  once_lanes_log2(n), st));
+        return REINA_RT_OK;
+    }
     HIP_TRY(hipMemsetAsync(s->fetch, 0, (kParts + 1) * kLine * 4, st));
     TraceInput tin{nullptr, 0, n, s->fetch, s->fetch + kParts * kLine};
     if (h16)
@@ -772,6 +792,11 @@ int reina_rt_intersect_noalloc(ReinaScene* s, const ReinaRay* rays, ReinaHit* hi
     int rc = scratch_address(s->device, &fetch);
     if (rc) return rc;
     if (n == 0) return REINA_RT_OK;
+    if (n <= kOnceRays) {
+        HIP_TRY(launch_trace_once(s->sv, (const float4*)rays, (float4*)hits, n, nullptr, false, s->tune.stack_depth,
+                                  once_lanes_log2(n), st));
+        return REINA_RT_OK;
+    }
     // the claim counters start at zero: a fill kernel, not hipMemsetAsync, so
     // the call can be captured in a HIP graph
     hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(256), 0, st, fetch, kNoAllocScratchWords);

@@ -224,6 +224,13 @@ hipError_t launch_trace(const SceneView& sv, const float4* rays, float4* hits, c
                      : launch_trace_f32(sv, rays, hits, in, stats, counters, count, tu, st);
 }
 
+hipError_t launch_trace_once(const SceneView& sv, const float4* rays, float4* hits, uint32_t n, uint32_t* counters,
+                             bool h16, uint32_t stack_depth, uint32_t lanes_log2, hipStream_t st) {
+    if (n == 0) return hipSuccess;
+    return sv.qnodes ? launch_trace_once_q8(sv, rays, hits, n, counters, stack_depth, lanes_log2, st)
+                     : launch_trace_once_f32(sv, rays, hits, n, counters, h16, stack_depth, lanes_log2, st);
+}
+
 hipError_t launch_shade(const SceneView& sv, const TraceParams& P, const PathState& S, const Queues& Q,
                         uint32_t in_q, Ctrl* ctrl, uint32_t slot, uint32_t grid, bool nee, hipStream_t st) {
     // k_shade needs a whole number (>= 1) of blocks per partition

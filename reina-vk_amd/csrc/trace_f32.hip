@@ -39,4 +39,13 @@ hipError_t launch_connect_f32(const SceneView& sv, const Queues& Q, const PathSt
     return launch_connect_fmt<false>(sv, Q, S, ctrl, slot, stats, tu, st);
 }
 
+hipError_t launch_trace_once_f32(const SceneView& sv, const float4* rays, float4* hits, uint32_t n, uint32_t* counters,
+                                 bool h16, uint32_t stack_depth, uint32_t lanes_log2, hipStream_t st) {
+    if (h16)
+        return counters ? launch_trace_once_fmt<false, true, true>(sv, rays, hits, n, counters, stack_depth, lanes_log2, st)
+                        : launch_trace_once_fmt<false, false, true>(sv, rays, hits, n, counters, stack_depth, lanes_log2, st);
+    return counters ? launch_trace_once_fmt<false, true, false>(sv, rays, hits, n, counters, stack_depth, lanes_log2, st)
+                    : launch_trace_once_fmt<false, false, false>(sv, rays, hits, n, counters, stack_depth, lanes_log2, st);
+}
+
 }  // namespace rt

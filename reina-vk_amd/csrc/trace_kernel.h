@@ -207,6 +207,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) vo
     }
 }
 
+// Closest-hit kernel for batches that fit the GPU at once: one ray per lane,
+// 1 << lanes_log2 rays per wave, no queue. Bound by the latency of the longest
+// ray's steps (about 50 us in a 327,686-triangle scene, however few the rays).
+template <int SD, bool COUNT, bool Q, bool H16>
+__global__ __launch_bounds__(256) void k_trace_once(SceneView sv, const float4* __restrict__ rays,
+                                                    float4* __restrict__ hits, uint32_t n, uint32_t* counters,
+                                                    uint32_t lanes_log2) {
+    __shared__ uint2 stack[SD * 256];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t i = ((blockIdx.x * 4u + (threadIdx.x >> 6)) << lanes_log2) + lane;
+    if ((lane >> lanes_log2) != 0u || i >= n) return;   // no barrier below
+    const void* nodes = Q ? static_cast<const void*>(sv.qnodes) : static_cast<const void*>(sv.nodes);
+    TRay r;
+    tray_init<H16>(r, rays[2 * i], rays[2 * i + 1]);
+    HitRec h = miss_record(r);
+    TravState ts;
+    trav_begin(ts);
+    uint32_t nv = 0, nt = 0;
+    bool active = r.valid && sv.num_nodes != 0;
+    while (active) active = trav_step<COUNT, Q, false, H16>(nodes, sv.tris, r, h, ts, stack + threadIdx.x, 256, nv, nt);
+    hits[i] = make_float4(h.t, __uint_as_float(h.prim), h.u, h.v);
+    if (COUNT && counters) { counters[2 * i] = nv; counters[2 * i + 1] = nt; }
+}
+
+template <bool Q, bool COUNT, bool H16>
+static hipError_t launch_trace_once_fmt(const SceneView& sv, const float4* rays, float4* hits, uint32_t n,
+                                        uint32_t* counters, uint32_t stack_depth, uint32_t lanes_log2, hipStream_t st) {
+    const uint32_t waves = (n + (1u << lanes_log2) - 1u) >> lanes_log2;
+    const dim3 g((waves + 3u) / 4u), b(256);
+    switch (stack_depth) {
+        case 8: hipLaunchKernelGGL((k_trace_once<8, COUNT, Q, H16>), g, b, 0, st, sv, rays, hits, n, counters, lanes_log2); break;
+        case 16: hipLaunchKernelGGL((k_trace_once<16, COUNT, Q, H16>), g, b, 0, st, sv, rays, hits, n, counters, lanes_log2); break;
+        case 24: hipLaunchKernelGGL((k_trace_once<24, COUNT, Q, H16>), g, b, 0, st, sv, rays, hits, n, counters, lanes_log2); break;
+        default: hipLaunchKernelGGL((k_trace_once<32, COUNT, Q, H16>), g, b, 0, st, sv, rays, hits, n, counters, lanes_log2); break;
+    }
+    return hipGetLastError();
+}
+
 template <bool Q, bool MULTI, int SD, int WAVES>
 static void launch_trace_sdw(const SceneView& sv, const float4* rays, float4* hits, const TraceInput& in,
                              unsigned long long* stats, uint32_t* counters, bool count, const Tuning& tu,

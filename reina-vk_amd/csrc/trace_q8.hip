@@ -14,4 +14,10 @@ hipError_t launch_connect_q8(const SceneView& sv, const Queues& Q, const PathSta
     return launch_connect_fmt<true>(sv, Q, S, ctrl, slot, stats, tu, st);
 }
 
+hipError_t launch_trace_once_q8(const SceneView& sv, const float4* rays, float4* hits, uint32_t n, uint32_t* counters,
+                                uint32_t stack_depth, uint32_t lanes_log2, hipStream_t st) {
+    return counters ? launch_trace_once_fmt<true, true, false>(sv, rays, hits, n, counters, stack_depth, lanes_log2, st)
+                    : launch_trace_once_fmt<true, false, false>(sv, rays, hits, n, counters, stack_depth, lanes_log2, st);
+}
+
 }  // namespace rt

@@ -121,6 +121,14 @@ struct TraceInput {
 // counters (optional, counting): per-ray {visits, tests}.
 hipError_t launch_trace(const SceneView& sv, const float4* rays, float4* hits, const TraceInput& in,
                         unsigned long long* stats, uint32_t* counters, bool count, const Tuning& tu, hipStream_t st);
+// Closest hits of n rays without a queue, 1 << lanes_log2 rays per wave.
+// counters != null: the counting build; h16 (FP32 nodes only): FP16 inverses.
+hipError_t launch_trace_once(const SceneView& sv, const float4* rays, float4* hits, uint32_t n, uint32_t* counters,
+                             bool h16, uint32_t stack_depth, uint32_t lanes_log2, hipStream_t st);
+hipError_t launch_trace_once_f32(const SceneView& sv, const float4* rays, float4* hits, uint32_t n, uint32_t* counters,
+                                 bool h16, uint32_t stack_depth, uint32_t lanes_log2, hipStream_t st);
+hipError_t launch_trace_once_q8(const SceneView& sv, const float4* rays, float4* hits, uint32_t n, uint32_t* counters,
+                                uint32_t stack_depth, uint32_t lanes_log2, hipStream_t st);
 // Closest hit of partitioned queue entries that belong to several requests
 // (pix: the queue's slot | request words).
 hipError_t launch_trace_multi(bool quantized, const float4* rays, float4* hits, const TraceInput& in,
