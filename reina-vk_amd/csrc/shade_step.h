@@ -12,6 +12,7 @@ namespace rt {
 struct ShadeResult {
     bool push;      // a next ray (no, nd) continues this pixel's path or starts its next sample
     bool finished;  // the pixel has finished all its samples
+    bool ended;     // a sample ended
     V3 no, nd;
     // next-event estimation: a shadow ray (so, sd, [0, stmax]) whose light,
     // if unoccluded, adds scontrib to the pixel's radiance
@@ -78,13 +79,19 @@ RT_D float light_pdf(float pdf_area, float d, V3 ng, V3 w, bool cull) {
     return cl > 0.0f ? (pdf_area * (d * d)) / cl : 0.0f;
 }
 
-// pp: index of the pixel's path state; px: pixel index in its image (y * W + x).
-// NEE: next-event estimation with MIS; S.st4 holds the last Lambertian bounce
+// A path's state (PathState) in registers; s4 with next-event estimation only.
+struct PathRegs {
+    uint4 s0;
+    float4 s1, s2, s3, s4;
+};
+
+// px: pixel index in its image (y * W + x).
+// NEE: next-event estimation with MIS; s4 holds the last Lambertian bounce
 // (its continuation ray's origin and the cosine pdf of that direction; 0
 // when the continuation is not MIS-weighted).
 template <bool NEE>
-RT_D ShadeResult shade_ray(const SceneView& sv, const TraceParams& P, const PathState& S, uint32_t pp,
-                           uint32_t px, float4 ra, float4 rb, float4 hh) {
+RT_D ShadeResult shade_path(const SceneView& sv, const TraceParams& P, PathRegs& T, uint32_t px, float4 ra, float4 rb,
+                            float4 hh) {
     ShadeResult r;
     r.push = false;
     r.shadow = false;
@@ -97,15 +104,15 @@ RT_D ShadeResult shade_ray(const SceneView& sv, const TraceParams& P, const Path
     // NEE code is compiled in with NEE and runs for requests that ask for it
     const bool nee = NEE && P.nee != 0u;
     float4 s4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (nee) s4 = S.st4[pp];
+    if (nee) s4 = T.s4;
     bool lambert_hit = false, disney_hit = false, emissive_mis = false;
     DisneyNee dn;
     const ReinaInstanceProperties* hp = nullptr;
     const MaterialRec RT_GLOBAL* hm = nullptr;
     V3 nee_n = r.no, nee_albedo = r.no;
     float emis_w = 1.0f;
-    uint4 s0 = S.st0[pp];
-    float4 s1 = S.st1[pp], s2 = S.st2[pp], s3 = S.st3[pp];
+    const uint4 s0 = T.s0;
+    const float4 s1 = T.s1, s2 = T.s2, s3 = T.s3;
     V3 O = v3(ra.x, ra.y, ra.z), D = v3(rb.x, rb.y, rb.z);
     Payload pld;
     pld.rng = s0.x;
@@ -257,17 +264,42 @@ RT_D ShadeResult shade_ray(const SceneView& sv, const TraceParams& P, const Path
             s4.w = 0.0f;
             r.push = true;
         }
-        S.st3[pp] = make_float4(sum.x, sum.y, sum.z, __uint_as_float(actual));
+        T.s3 = make_float4(sum.x, sum.y, sum.z, __uint_as_float(actual));
     } else {
         r.no = pld.rayOrigin;
         r.nd = pld.rayDirection;
         r.push = true;
     }
-    S.st0[pp] = make_uint4(pld.rng, sample, seg, pld.insideDielectric ? 1u : 0u);
-    S.st1[pp] = make_float4(thr.x, thr.y, thr.z, pld.accumulatedDistance);
-    S.st2[pp] = make_float4(L.x, L.y, L.z, 0.0f);
-    if (nee) S.st4[pp] = s4;
+    T.s0 = make_uint4(pld.rng, sample, seg, pld.insideDielectric ? 1u : 0u);
+    T.s1 = make_float4(thr.x, thr.y, thr.z, pld.accumulatedDistance);
+    T.s2 = make_float4(L.x, L.y, L.z, 0.0f);
+    if (nee) T.s4 = s4;
     r.finished = !r.push;
+    r.ended = end;
+    return r;
+}
+
+RT_D void load_path(PathRegs& T, const PathState& S, uint32_t pp) {
+    T.s0 = S.st0[pp];
+    T.s1 = S.st1[pp];
+    T.s2 = S.st2[pp];
+    T.s3 = S.st3[pp];
+}
+
+// shade_path on the path state in memory; pp: its index.
+template <bool NEE>
+RT_D ShadeResult shade_ray(const SceneView& sv, const TraceParams& P, const PathState& S, uint32_t pp,
+                           uint32_t px, float4 ra, float4 rb, float4 hh) {
+    PathRegs T;
+    load_path(T, S, pp);
+    const bool nee = NEE && P.nee != 0u;
+    if (nee) T.s4 = S.st4[pp];
+    const ShadeResult r = shade_path<NEE>(sv, P, T, px, ra, rb, hh);
+    if (r.ended) S.st3[pp] = T.s3;
+    S.st0[pp] = T.s0;
+    S.st1[pp] = T.s1;
+    S.st2[pp] = T.s2;
+    if (nee) S.st4[pp] = T.s4;
     return r;
 }
 
