@@ -675,63 +675,107 @@ RT_D float4 unorm8(uint32_t t) {
     return make_float4(over255(t & 0xFFu), over255((t >> 8) & 0xFFu), over255((t >> 16) & 0xFFu), over255(t >> 24));
 }
 
-// floor(x) mod n for a floored, finite x with |x| <= 2^30; coordinates in
-// (or within one texture of) the unit square, which is where uv mod 1 and a
-// bump search's steps lie, take no integer division
-RT_D uint32_t repeat_index(float fx, uint32_t n) {
+// i0 = floor(x) mod n and i1 = (floor(x) + 1) mod n for a floored, finite x = fx
+// with |x| <= 2^30; coordinates in (or within one texture of) the unit square,
+// which is where uv mod 1 and a bump search's steps lie, take no integer
+// division
+RT_D void repeat_pair(float fx, uint32_t n, uint32_t& i0, uint32_t& i1) {
     const int32_t i = (int32_t)fx, w = (int32_t)n;
     int32_t m = i < 0 ? i + w : (i >= w ? i - w : i);
+    int32_t m1 = m + 1 == w ? 0 : m + 1;
     if ((uint32_t)m >= n) {
         m = i % w;
         m = m < 0 ? m + w : m;
+        m1 = (int32_t)(fx + 1.0f) % w;   // beyond 2^24, fx + 1 is fx
+        m1 = m1 < 0 ? m1 + w : m1;
     }
-    return (uint32_t)m;
+    i0 = (uint32_t)m;
+    i1 = (uint32_t)m1;
 }
 
-RT_D float4 tex_sample(const SceneView& sv, int32_t id, float u, float v) {
-    const TexInfo t = sv.tex[id];
+// The four texels around (u, v) and the weights between them.
+struct TexTaps {
+    uint32_t t00, t10, t01, t11;
+    float a, b;
+};
+RT_D TexTaps tex_taps(const TexInfo& t, const uint32_t RT_GLOBAL* texels, float u, float v) {
     float x = u * (float)t.w - 0.5f, y = v * (float)t.h - 0.5f;
     // non-finite coordinates (a NaN uv) read texel 0; huge ones are clamped so
     // the integer conversion stays defined
     x = (x == x) ? clampf_(x, -1073741824.0f, 1073741824.0f) : 0.0f;
     y = (y == y) ? clampf_(y, -1073741824.0f, 1073741824.0f) : 0.0f;
     const float fx = floorf(x), fy = floorf(y);
-    const float a = x - fx, b = y - fy;
-    const uint32_t i0 = repeat_index(fx, t.w), i1 = repeat_index(fx + 1.0f, t.w);
-    const uint32_t j0 = repeat_index(fy, t.h), j1 = repeat_index(fy + 1.0f, t.h);
-    const uint32_t* row0 = sv.texels + t.base + (uint64_t)j0 * t.w;
-    const uint32_t* row1 = sv.texels + t.base + (uint64_t)j1 * t.w;
-    const float4 t00 = unorm8(row0[i0]), t10 = unorm8(row0[i1]), t01 = unorm8(row1[i0]), t11 = unorm8(row1[i1]);
-    // two linear interpolations along x, then one along y: exact for equal texels
-    const auto lerp2 = [a, b](float p00, float p10, float p01, float p11) {
-        const float top = p00 + a * (p10 - p00), bottom = p01 + a * (p11 - p01);
-        return top + b * (bottom - top);
-    };
-    return make_float4(lerp2(t00.x, t10.x, t01.x, t11.x), lerp2(t00.y, t10.y, t01.y, t11.y),
-                       lerp2(t00.z, t10.z, t01.z, t11.z), lerp2(t00.w, t10.w, t01.w, t11.w));
+    uint32_t i0, i1, j0, j1;
+    repeat_pair(fx, t.w, i0, i1);
+    repeat_pair(fy, t.h, j0, j1);
+    const uint32_t r0 = j0 * t.w, r1 = j1 * t.w;   // below 2^32: at most 65536 x 65536 texels
+    TexTaps p;
+    p.a = x - fx;
+    p.b = y - fy;
+    const uint32_t RT_GLOBAL* base = texels + t.base;
+    p.t00 = base[r0 + i0];
+    p.t10 = base[r0 + i1];
+    p.t01 = base[r1 + i0];
+    p.t11 = base[r1 + i1];
+    return p;
+}
+// two linear interpolations along x, then one along y: exact for equal texels
+RT_D float tex_lerp(const TexTaps& p, float p00, float p10, float p01, float p11) {
+    const float top = p00 + p.a * (p10 - p00), bottom = p01 + p.a * (p11 - p01);
+    return top + p.b * (bottom - top);
+}
+
+RT_D float4 tex_sample(const SceneView& sv, int32_t id, float u, float v) {
+    const TexTaps p = tex_taps(sv.tex[id], sv.texels, u, v);
+    const float4 t00 = unorm8(p.t00), t10 = unorm8(p.t10), t01 = unorm8(p.t01), t11 = unorm8(p.t11);
+    return make_float4(tex_lerp(p, t00.x, t10.x, t01.x, t11.x), tex_lerp(p, t00.y, t10.y, t01.y, t11.y),
+                       tex_lerp(p, t00.z, t10.z, t01.z, t11.z), tex_lerp(p, t00.w, t10.w, t01.w, t11.w));
 }
 
 // texutils.h.glsl:4-41 (parallax occlusion search). The layer loop ends
-// within 0.2 * 512 + 1 steps for finite input; the cap only guards NaN.
-constexpr int kBumpMaxSteps = 1024;
+// within 0.2 * 512 + 1 steps for finite input; the cap only guards NaN. A
+// layer's position does not depend on the heights found, so the heights of the
+// next kBumpAhead layers are fetched together: one at a time, each of a
+// search's up to 102 layers waited for its texels in turn.
+constexpr int kBumpMaxSteps = 1024, kBumpAhead = 4;
 RT_D void bump_mapping(const SceneView& sv, int32_t id, float& u, float& v, V3 rayIn, const M3& T) {
     const float heightScale = 0.2f, minLayers = 64.0f, maxLayers = 512.0f;
     const V3 V = normalize(tmul(T, neg(rayIn)));
     if (V.z <= 0.0f) return;
     const float numLayers = mixf(maxLayers, minLayers, clampf_(V.z, 0.0f, 1.0f));
-    const float layerDepth = 1.0f / numLayers;
+    const float layerDepth = inv_(numLayers);
     const float Px = V.x / V.z * heightScale, Py = V.y / V.z * heightScale;
     const float du = Px / numLayers, dv = Py / numLayers;
+    const TexInfo tex = sv.tex[id];
+    const uint32_t RT_GLOBAL* texels = sv.texels;
+    const auto height = [&](const TexTaps& p) {
+        return tex_lerp(p, over255(p.t00 & 0xFFu), over255(p.t10 & 0xFFu), over255(p.t01 & 0xFFu),
+                        over255(p.t11 & 0xFFu)) * heightScale;
+    };
     float cu = u, cv = v, depthSum = 0.0f;
-    float h = tex_sample(sv, id, cu, cv).x * heightScale;
-    for (int k = 0; k < kBumpMaxSteps && depthSum < h; ++k) {
-        cu = cu - du;
-        cv = cv - dv;
-        depthSum = depthSum + layerDepth;
-        h = tex_sample(sv, id, cu, cv).x * heightScale;
+    float h = height(tex_taps(tex, texels, cu, cv));
+    for (int k = 0; k < kBumpMaxSteps && depthSum < h;) {
+        float us[kBumpAhead], vs[kBumpAhead];
+        TexTaps p[kBumpAhead];
+#pragma unroll
+        for (int q = 0; q < kBumpAhead; ++q) {
+            us[q] = (q ? us[q - 1] : cu) - du;
+            vs[q] = (q ? vs[q - 1] : cv) - dv;
+            p[q] = tex_taps(tex, texels, us[q], vs[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < kBumpAhead; ++q) {
+            if (k < kBumpMaxSteps && depthSum < h) {
+                cu = us[q];
+                cv = vs[q];
+                depthSum = depthSum + layerDepth;
+                h = height(p[q]);
+                ++k;
+            }
+        }
     }
     const float pu = cu + du, pv = cv + dv;
-    const float hPrev = tex_sample(sv, id, pu, pv).x * heightScale;
+    const float hPrev = height(tex_taps(tex, texels, pu, pv));
     const float sumPrev = depthSum - layerDepth;
     const float after = h - depthSum;
     const float before = hPrev - sumPrev;
