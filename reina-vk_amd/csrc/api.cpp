@@ -3,7 +3,7 @@
 // reina_rt_scene_create  replaces Scene::build's BLAS/TLAS construction
 //                        (src/scene/Scene.cpp:93-116): validate the packed
 //                        Models/Instances buffers, flatten every instance to
-//                        world space, build the BVH8, upload one HBM arena.
+//                        world space and build the BVH8 in HBM.
 // reina_rt_trace         replaces Reina::traceRays' vkCmdTraceRaysKHR
 //                        (src/Reina.cpp:425-470): init, then extend/shade
 //                        bounce iterations until every pixel has finished its
@@ -46,6 +46,22 @@ int reina_rt_abi_version(uint32_t* version, uint32_t* s_ip, uint32_t* s_pc, uint
 
 const char* reina_rt_last_error(void) { return g_err.c_str(); }
 
+// The first of n values that is not below limit, or n. Blocks are checked
+// without an exit in their loop, so that it is vectorised.
+static uint64_t first_out_of_range(const uint32_t* p, uint64_t n, uint64_t limit) {
+    if (limit > 0xFFFFFFFFull) return n;
+    const uint32_t lim = (uint32_t)limit;
+    for (uint64_t b = 0; b < n; b += 4096) {
+        const uint64_t e = std::min<uint64_t>(n, b + 4096);
+        uint32_t bad = 0;
+        for (uint64_t i = b; i < e; ++i) bad |= p[i] >= lim ? 1u : 0u;
+        if (!bad) continue;
+        while (p[b] < lim) ++b;
+        return b;
+    }
+    return n;
+}
+
 static int validate(const ReinaSceneDesc* d) {
     if (!d) return fail(REINA_RT_ERR_INVALID_ARG, "scene description is null");
     if (d->struct_size != sizeof(ReinaSceneDesc))
@@ -62,12 +78,12 @@ static int validate(const ReinaSceneDesc* d) {
         if ((uint64_t)r.indexOffset + 3ull * r.indexCount > d->num_indices)
             return fail(REINA_RT_ERR_INVALID_ARG, "model " + std::to_string(m) + " index range exceeds indices");
     }
-    for (uint64_t i = 0; i < d->num_indices; ++i)
-        if (d->indices[i] >= d->num_vertices)
-            return fail(REINA_RT_ERR_INVALID_ARG, "index " + std::to_string(i) + " out of vertex range");
-    for (uint64_t i = 0; i < d->num_tbn_indices; ++i)
-        if (d->tbn_indices[i] >= d->num_tbns)
-            return fail(REINA_RT_ERR_INVALID_ARG, "tbn index " + std::to_string(i) + " out of range");
+    uint64_t bad = first_out_of_range(d->indices, d->num_indices, d->num_vertices);
+    if (bad < d->num_indices)
+        return fail(REINA_RT_ERR_INVALID_ARG, "index " + std::to_string(bad) + " out of vertex range");
+    bad = first_out_of_range(d->tbn_indices, d->num_tbn_indices, d->num_tbns);
+    if (bad < d->num_tbn_indices)
+        return fail(REINA_RT_ERR_INVALID_ARG, "tbn index " + std::to_string(bad) + " out of range");
     // texture-coordinate indices are read only through an instance whose
     // texIndicesOffset is set: a model without UVs (texIndexOffset = -1,
     // Models.cpp:50) keeps index values with no coordinates behind them
@@ -115,7 +131,7 @@ static void set_normal_matrix(InstanceRec& r) {
     const V3 n[3] = {scale(cross(c1, c2), invdet), scale(cross(c2, c0), invdet), scale(cross(c0, c1), invdet)};
     float* out[3] = {r.n0, r.n1, r.n2};
     for (int k = 0; k < 3; ++k) { out[k][0] = n[k].x; out[k][1] = n[k].y; out[k][2] = n[k].z; }
-    r.pad[0] = r.pad[1] = r.pad[2] = 0.0f;
+    r.pad[0] = r.pad[1] = 0.0f;
 }
 
 // The operations of evalDisney's and sampleDisney's weights and GGX alphas
@@ -134,14 +150,22 @@ static MaterialRec make_material(const ReinaInstanceProperties& p) {
     return m;
 }
 
-// Light-sampling tables (EmissiveInst, rt_layout.h) from the flattened
-// world-space triangles, in double precision.
-static void build_emissive(ReinaScene* s, const ReinaSceneDesc* d, const std::vector<InstanceRec>& inst,
-                           const std::vector<float>& wtri) {
+// One triangle in world space: ((c0*x + c1*y) + c2*z) + c3 for each corner.
+static void world_triangle(const ReinaSceneDesc* d, const InstanceRec& r, uint32_t prim, float* out) {
+    for (int k = 0; k < 3; ++k) {
+        const uint32_t vi = d->indices[3ull * prim + r.index_offset + k];
+        const float x = d->vertices[4ull * vi], y = d->vertices[4ull * vi + 1], z = d->vertices[4ull * vi + 2];
+        for (int c = 0; c < 3; ++c) out[3 * k + c] = ((r.c0[c] * x + r.c1[c] * y) + r.c2[c] * z) + r.c3[c];
+    }
+}
+
+// Light-sampling tables (EmissiveInst, rt_layout.h) from the world-space
+// triangles, in double precision.
+static void build_emissive(ReinaScene* s, const ReinaSceneDesc* d, const std::vector<InstanceRec>& inst, uint64_t num_tris) {
     s->emi.clear();
     s->tri_cdf.clear();
     s->inst_emi.assign(inst.size(), -1);
-    s->tri_flags.assign(wtri.size() / 9, 0);
+    s->tri_flags.assign(num_tris, 0);
     std::vector<double> weight;
     double total = 0.0;
     for (uint32_t i = 0; i < inst.size(); ++i) {
@@ -159,7 +183,8 @@ static void build_emissive(ReinaScene* s, const ReinaSceneDesc* d, const std::ve
         std::vector<double> cum(ntri);
         double area = 0.0;
         for (uint32_t t = 0; t < ntri; ++t) {
-            const float* w = &wtri[9ull * (r.tri_base + t)];
+            float w[9];
+            world_triangle(d, r, t, w);
             double ax = (double)w[3] - w[0], ay = (double)w[4] - w[1], az = (double)w[5] - w[2];
             double bx = (double)w[6] - w[0], by = (double)w[7] - w[1], bz = (double)w[8] - w[2];
             double cx = ay * bz - az * by, cy = az * bx - ax * bz, cz = ax * by - ay * bx;
@@ -188,9 +213,10 @@ static void build_emissive(ReinaScene* s, const ReinaSceneDesc* d, const std::ve
     if (!s->emi.empty()) s->emi.back().cdf = 1.0f;
 }
 
-static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vector<float>& wtri,
-                        const std::vector<uint32_t>& tri_inst, const std::vector<uint32_t>& tri_prim,
-                        const std::vector<InstanceRec>& inst) {
+// Everything but the tree; the tree's build fills the ids of the triangles
+// (mesh), and scene_finish what is derived from them.
+static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vector<InstanceRec>& inst, uint32_t num_tris,
+                        DeviceMesh& mesh, float4*& rec) {
     auto al = [](uint64_t x) { return (x + 255) & ~255ull; };
     struct Part { const void* src; uint64_t bytes; uint64_t off; };
     std::vector<Part> parts;
@@ -200,11 +226,8 @@ static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vecto
         off += al(bytes ? bytes : 4);
         return parts.size() - 1;
     };
-    size_t p_nodes = s->quantized ? add(s->host_qnodes.data(), s->host_qnodes.size() * sizeof(QBvh8Node))
-                                  : add(s->host_nodes.data(), s->host_nodes.size() * sizeof(Bvh8Node));
-    size_t p_tris = add(s->host_tris.data(), s->host_tris.size() * sizeof(float));
-    size_t p_ti = add(tri_inst.data(), tri_inst.size() * 4);
-    size_t p_tp = add(tri_prim.data(), tri_prim.size() * 4);
+    size_t p_ti = add(nullptr, num_tris * 4ull);   // these two filled on the device
+    size_t p_tp = add(nullptr, num_tris * 4ull);
     size_t p_in = add(inst.data(), inst.size() * sizeof(InstanceRec));
     size_t p_pr = add(d->props, (uint64_t)d->num_props * sizeof(ReinaInstanceProperties));
     std::vector<MaterialRec> mats(d->num_props);
@@ -220,7 +243,7 @@ static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vecto
     size_t p_cdf = add(s->tri_cdf.data(), s->tri_cdf.size() * 4);
     size_t p_ie = add(s->inst_emi.data(), s->inst_emi.size() * 4);
     size_t p_tf = add(s->tri_flags.data(), s->tri_flags.size());
-    size_t p_rec = add(nullptr, tri_inst.size() * (uint64_t)kShadeRecF4 * 16);   // filled on the device
+    size_t p_rec = add(nullptr, num_tris * (uint64_t)kShadeRecF4 * 16);   // filled on the device
     // textures: a TexInfo table, then every texture's texels (RGBA8 packed in 32 bits)
     std::vector<TexInfo> tinfo(d->num_textures);
     uint64_t ntexel = 0;
@@ -230,20 +253,16 @@ static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vecto
     }
     size_t p_tinfo = add(tinfo.data(), tinfo.size() * sizeof(TexInfo));
     size_t p_texel = add(nullptr, ntexel * 4);
-    (void)wtri;
     HIP_TRY(hipSetDevice(s->device));
     hipError_t e = hipMalloc(&s->arena, off);
     if (e != hipSuccess) return fail(REINA_RT_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(off) + " bytes failed");
-    s->arena_bytes = off;
+    s->info.device_bytes = off;
     for (const Part& p : parts)
         if (p.bytes && p.src) HIP_TRY(hipMemcpy((char*)s->arena + p.off, p.src, p.bytes, hipMemcpyHostToDevice));
     char* a = (char*)s->arena;
     for (uint32_t t = 0; t < d->num_textures; ++t)   // byte order r, g, b, a = the packed word's low to high byte
         HIP_TRY(hipMemcpy(a + parts[p_texel].off + 4 * tinfo[t].base, d->textures[t].rgba8,
                           4ull * tinfo[t].w * tinfo[t].h, hipMemcpyHostToDevice));
-    s->sv.nodes = s->quantized ? nullptr : (const Bvh8Node RT_GLOBAL*)(a + parts[p_nodes].off);
-    s->sv.qnodes = s->quantized ? (const QBvh8Node RT_GLOBAL*)(a + parts[p_nodes].off) : nullptr;
-    s->sv.tris = (const float4 RT_GLOBAL*)(a + parts[p_tris].off);
     s->sv.tri_inst = (const uint32_t RT_GLOBAL*)(a + parts[p_ti].off);
     s->sv.tri_prim = (const uint32_t RT_GLOBAL*)(a + parts[p_tp].off);
     s->sv.inst = (const InstanceRec RT_GLOBAL*)(a + parts[p_in].off);
@@ -258,8 +277,7 @@ static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vecto
     s->sv.num_tbns = d->num_tbns;
     s->sv.num_tbn_indices = d->num_tbn_indices;
     s->sv.num_tex_coords = d->num_tex_coords;
-    s->sv.num_nodes = s->host_nodes.size();
-    s->sv.num_tris = tri_inst.size();
+    s->sv.num_tris = num_tris;
     s->sv.emi = (const EmissiveInst RT_GLOBAL*)(a + parts[p_emi].off);
     s->sv.tri_cdf = (const float RT_GLOBAL*)(a + parts[p_cdf].off);
     s->sv.inst_emi = (const int32_t RT_GLOBAL*)(a + parts[p_ie].off);
@@ -269,10 +287,87 @@ static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vecto
     s->sv.tex = (const TexInfo RT_GLOBAL*)(a + parts[p_tinfo].off);
     s->sv.texels = (const uint32_t RT_GLOBAL*)(a + parts[p_texel].off);
     s->sv.num_tex = d->num_textures;
-    float4* rec = (float4*)(a + parts[p_rec].off);
-    HIP_TRY(launch_shade_records(s->sv, rec, (uint32_t)tri_inst.size(), nullptr));
-    HIP_TRY(hipStreamSynchronize(nullptr));
+    rec = (float4*)(a + parts[p_rec].off);
     s->sv.srec = (const float4 RT_GLOBAL*)rec;
+    mesh.inst = (const InstanceRec*)(a + parts[p_in].off);
+    mesh.vertices = (const float4*)(a + parts[p_v].off);
+    mesh.indices = (const uint32_t*)(a + parts[p_i].off);
+    mesh.tri_inst = (uint32_t*)(a + parts[p_ti].off);
+    mesh.tri_prim = (uint32_t*)(a + parts[p_tp].off);
+    mesh.num_inst = (uint32_t)inst.size();
+    mesh.num_tris = num_tris;
+    return REINA_RT_OK;
+}
+
+// The tree into an allocation of its size.
+static int scene_set_tree(ReinaScene* s, const void* nodes, hipMemcpyKind nodes_from, uint64_t num_nodes,
+                          const void* tris, hipMemcpyKind tris_from, uint64_t num_tris) {
+    const uint64_t nb = num_nodes * (s->quantized ? sizeof(QBvh8Node) : sizeof(Bvh8Node)), tb = num_tris * 48;
+    auto al = [](uint64_t x) { return ((x ? x : 4) + 255) & ~255ull; };
+    if (hipMalloc(&s->tree, al(nb) + al(tb)) != hipSuccess)
+        return fail(REINA_RT_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(al(nb) + al(tb)) + " bytes failed");
+    s->tree_tris = al(nb);
+    s->info.device_bytes += al(nb) + al(tb);
+    char* t = (char*)s->tree;
+    HIP_TRY(hipMemcpyAsync(t, nodes, nb, nodes_from, nullptr));
+    if (tb) HIP_TRY(hipMemcpyAsync(t + s->tree_tris, tris, tb, tris_from, nullptr));
+    s->sv.nodes = s->quantized ? nullptr : (const Bvh8Node RT_GLOBAL*)t;
+    s->sv.qnodes = s->quantized ? (const QBvh8Node RT_GLOBAL*)t : nullptr;
+    s->sv.tris = (const float4 RT_GLOBAL*)(t + s->tree_tris);
+    s->sv.num_nodes = num_nodes;
+    return REINA_RT_OK;
+}
+
+// Builds the tree (its depth and cost to s->info) and finishes the scene.
+static int scene_build(ReinaScene* s, const ReinaSceneDesc* d, const std::vector<InstanceRec>& inst, uint64_t num_tris) {
+    auto flatten = [&](std::vector<float>& w) {
+        w.resize(9 * num_tris);
+        for (const InstanceRec& r : inst)
+            for (uint32_t p = 0; p < d->models[r.model].indexCount; ++p)
+                world_triangle(d, r, p, &w[9ull * (r.tri_base + p)]);
+    };
+    const bool on_host = (d->flags & REINA_RT_BUILD_HOST) != 0;   // the device build is the default
+    Bvh8Result host;
+    DeviceBvh dev;
+    std::string err;
+    if (on_host) {
+        std::vector<float> w;
+        flatten(w);
+        if (!build_bvh8_host(w.data(), num_tris, host, err)) return fail(REINA_RT_ERR_INVALID_ARG, err);
+    }
+    if (hipSetDevice(s->device) != hipSuccess) return fail(REINA_RT_ERR_DEVICE, "hipSetDevice failed");
+    build_emissive(s, d, inst, num_tris);
+    DeviceMesh mesh;
+    float4* rec = nullptr;
+    int rc = scene_upload(s, d, inst, (uint32_t)num_tris, mesh, rec);
+    if (rc) return rc;
+    if (on_host)
+        HIP_TRY(launch_triangle_ids(mesh, nullptr));
+    else if (!build_bvh8_device(mesh, flatten, dev, err))
+        return fail(REINA_RT_ERR_DEVICE, "device BVH build: " + err);
+    s->info.max_depth = on_host ? host.max_depth : dev.max_depth;
+    s->info.sah_cost = on_host ? host.sah_cost : dev.sah_cost;
+    if (s->info.max_depth > kMaxStackDepth + 1)
+        return fail(REINA_RT_ERR_UNSUPPORTED, "BVH8 depth " + std::to_string(s->info.max_depth) +
+                                                  " exceeds the traversal stack (" + std::to_string(kMaxStackDepth) + ")");
+    const uint64_t num_nodes = on_host ? host.nodes.size() : dev.num_nodes;
+    const void* nodes = on_host ? (const void*)host.nodes.data() : dev.nodes;
+    std::vector<QBvh8Node> qnodes;
+    if (d->flags & REINA_RT_NODES_QUANTIZED) {
+        if (!on_host) {
+            host.nodes.resize(num_nodes);
+            HIP_TRY(hipMemcpy(host.nodes.data(), dev.nodes, num_nodes * sizeof(Bvh8Node), hipMemcpyDeviceToHost));
+        }
+        if (!quantize_bvh8(host.nodes, qnodes, err)) return fail(REINA_RT_ERR_INVALID_ARG, err);
+        s->quantized = true;
+        nodes = qnodes.data();
+    }
+    rc = scene_set_tree(s, nodes, on_host || s->quantized ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice, num_nodes,
+                        on_host ? (const void*)host.tris.data() : dev.tris,
+                        on_host ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice, num_tris);
+    if (rc) return rc;
+    HIP_TRY(launch_shade_records(s->sv, rec, (uint32_t)num_tris, nullptr));
+    HIP_TRY(hipStreamSynchronize(nullptr));
     return REINA_RT_OK;
 }
 
@@ -286,7 +381,6 @@ int reina_rt_scene_create(const ReinaSceneDesc* d, ReinaScene** out) {
         return fail(REINA_RT_ERR_DEVICE, "no HIP device available");
     if ((int)d->device >= ndev) return fail(REINA_RT_ERR_INVALID_ARG, "device ordinal out of range");
     auto t0 = std::chrono::steady_clock::now();
-    // flatten: world = ((c0*x + c1*y) + c2*z) + c3, instance-major order
     uint64_t ntri = 0;
     std::vector<InstanceRec> inst(d->num_instances);
     for (uint32_t i = 0; i < d->num_instances; ++i) {
@@ -298,79 +392,31 @@ int reina_rt_scene_create(const ReinaSceneDesc* d, ReinaScene** out) {
         r.material = id.materialIdx;
         r.model = id.modelID;
         r.tri_base = (uint32_t)ntri;
+        r.index_offset = d->models[id.modelID].indexOffset;
         set_normal_matrix(r);
         ntri += d->models[id.modelID].indexCount;
     }
     if (ntri >= (1ull << 24)) return fail(REINA_RT_ERR_INVALID_ARG, "more than 2^24 triangles in one scene");
-    std::vector<float> wtri(9 * ntri);
-    std::vector<uint32_t> tri_inst(ntri), tri_prim(ntri);
-    for (uint32_t i = 0; i < d->num_instances; ++i) {
-        const InstanceRec& r = inst[i];
-        const ReinaModelRange& mr = d->models[r.model];
-        for (uint32_t p = 0; p < mr.indexCount; ++p) {
-            uint64_t g = (uint64_t)r.tri_base + p;
-            for (int k = 0; k < 3; ++k) {
-                uint32_t vi = d->indices[3ull * p + mr.indexOffset + k];
-                float x = d->vertices[4ull * vi], y = d->vertices[4ull * vi + 1], z = d->vertices[4ull * vi + 2];
-                for (int c = 0; c < 3; ++c)
-                    wtri[9 * g + 3 * k + c] = ((r.c0[c] * x + r.c1[c] * y) + r.c2[c] * z) + r.c3[c];
-            }
-            tri_inst[g] = i;
-            tri_prim[g] = p;
-        }
-    }
     ReinaScene* s = new ReinaScene();
     s->device = (int)d->device;
-    Bvh8Result bvh;
-    std::string err;
-    if (!(d->flags & REINA_RT_BUILD_HOST)) {   // the device build is the default
-        if (hipSetDevice(s->device) != hipSuccess) {
-            delete s;
-            return fail(REINA_RT_ERR_DEVICE, "hipSetDevice failed");
-        }
-        if (!build_bvh8_device(wtri.data(), ntri, bvh, err, &s->device_build_ms)) {
-            delete s;
-            return fail(REINA_RT_ERR_DEVICE, "device BVH build: " + err);
-        }
-    } else if (!build_bvh8_host(wtri.data(), ntri, bvh, err)) {
-        delete s;
-        return fail(REINA_RT_ERR_INVALID_ARG, err);
-    }
-    if (bvh.max_depth > kMaxStackDepth + 1) {
-        delete s;
-        return fail(REINA_RT_ERR_UNSUPPORTED, "BVH8 depth " + std::to_string(bvh.max_depth) +
-                                                  " exceeds the traversal stack (" + std::to_string(kMaxStackDepth) + ")");
-    }
-    s->host_nodes = std::move(bvh.nodes);
-    s->host_tris = std::move(bvh.tris);
-    if (d->flags & REINA_RT_NODES_QUANTIZED) {
-        if (!quantize_bvh8(s->host_nodes, s->host_qnodes, err)) {
-            delete s;
-            return fail(REINA_RT_ERR_INVALID_ARG, err);
-        }
-        s->quantized = true;
-    }
-    build_emissive(s, d, inst, wtri);
-    rc = scene_upload(s, d, wtri, tri_inst, tri_prim, inst);
+    rc = scene_build(s, d, inst, ntri);
     if (rc) {
+        if (s->tree) hipFree(s->tree);
         if (s->arena) hipFree(s->arena);
         delete s;
         return rc;
     }
     auto t1 = std::chrono::steady_clock::now();
     s->info.num_triangles = ntri;
-    s->info.num_nodes = s->host_nodes.size();
+    s->info.num_nodes = s->sv.num_nodes;
     s->info.node_bytes = s->quantized ? sizeof(QBvh8Node) : sizeof(Bvh8Node);
-    s->info.device_bytes = s->arena_bytes;
-    s->info.max_depth = bvh.max_depth;
     s->info.quantized = s->quantized ? 1u : 0u;
     s->info.num_emissive = (uint32_t)s->emi.size();
     s->info.build_ms = std::chrono::duration<float, std::milli>(t1 - t0).count();
-    s->info.sah_cost = bvh.sah_cost;
     hipDeviceProp_t prop;
     HIP_TRY(hipGetDeviceProperties(&prop, s->device));
     uint32_t cus = (uint32_t)prop.multiProcessorCount;
-    uint32_t need = bvh.max_depth > 1 ? bvh.max_depth - 1 : 1;
+    uint32_t need = s->info.max_depth > 1 ? s->info.max_depth - 1 : 1;
     s->tune.stack_depth = need <= 8 ? 8 : (need <= 16 ? 16 : (need <= 24 ? 24 : 32));
     s->tune.refill_min = 32;
     s->tune.grid = cus * (s->tune.stack_depth <= 8 ? 8 : 4);
@@ -401,6 +447,7 @@ int reina_rt_scene_destroy(ReinaScene* s) {
     for (int r = 0; r < 2; ++r)
         if (s->cev[r]) hipEventDestroy(s->cev[r]);
     for (hipEvent_t e : s->xev) hipEventDestroy(e);
+    if (s->tree) hipFree(s->tree);
     if (s->arena) hipFree(s->arena);
     delete s;
     return REINA_RT_OK;
@@ -412,19 +459,38 @@ int reina_rt_scene_info(const ReinaScene* s, ReinaSceneInfo* o) {
     return REINA_RT_OK;
 }
 
+// The tree, read back from HBM. A non-blocking stream of its own: the copy
+// neither waits for a caller's work nor takes part in a capture, also one of
+// another thread (the scene does not change after its creation).
+static int copy_from_scene(const ReinaScene* s, void* nodes, uint64_t nb, void* tris, uint64_t tb) {
+    int before = 0;
+    HIP_TRY(hipGetDevice(&before));
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+    hipStream_t st = nullptr;
+    hipError_t e = before == s->device ? hipSuccess : hipSetDevice(s->device);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+    if (e == hipSuccess && nodes) e = hipMemcpyAsync(nodes, s->tree, nb, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess && tris && tb)
+        e = hipMemcpyAsync(tris, (const char*)s->tree + s->tree_tris, tb, hipMemcpyDeviceToHost, st);
+    const hipError_t e2 = st ? hipStreamSynchronize(st) : hipSuccess;
+    if (st) (void)hipStreamDestroy(st);
+    if (before != s->device) (void)hipSetDevice(before);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    HIP_TRY(e);
+    HIP_TRY(e2);
+    return REINA_RT_OK;
+}
+
 int reina_rt_scene_export_bvh(const ReinaScene* s, void* nodes, uint64_t* nodes_bytes, void* tris,
                               uint64_t* tris_bytes) {
     if (!s || !nodes_bytes || !tris_bytes) return fail(REINA_RT_ERR_INVALID_ARG, "null argument");
-    const void* src = s->quantized ? (const void*)s->host_qnodes.data() : (const void*)s->host_nodes.data();
-    uint64_t nb = s->quantized ? s->host_qnodes.size() * sizeof(QBvh8Node) : s->host_nodes.size() * sizeof(Bvh8Node);
-    uint64_t tb = s->host_tris.size() * sizeof(float);
-    if (nodes) {
-        if (*nodes_bytes < nb) return fail(REINA_RT_ERR_INVALID_ARG, "nodes buffer too small");
-        std::memcpy(nodes, src, nb);
-    }
-    if (tris) {
-        if (*tris_bytes < tb) return fail(REINA_RT_ERR_INVALID_ARG, "tris buffer too small");
-        std::memcpy(tris, s->host_tris.data(), tb);
+    const uint64_t nb = s->sv.num_nodes * s->info.node_bytes, tb = s->info.num_triangles * 48ull;
+    if (nodes && *nodes_bytes < nb) return fail(REINA_RT_ERR_INVALID_ARG, "nodes buffer too small");
+    if (tris && *tris_bytes < tb) return fail(REINA_RT_ERR_INVALID_ARG, "tris buffer too small");
+    if ((nodes && nb) || (tris && tb)) {
+        int rc = copy_from_scene(s, nodes, nb, tris, tb);
+        if (rc) return rc;
     }
     *nodes_bytes = nb;
     *tris_bytes = tb;

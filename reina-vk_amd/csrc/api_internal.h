@@ -57,14 +57,11 @@ inline TraceParams make_trace_params(const RtPushConsts* pc, uint32_t W, uint32_
 struct ReinaScene {
     int device = 0;
     rt::SceneView sv{};
-    void* arena = nullptr;
-    uint64_t arena_bytes = 0;
+    void* arena = nullptr;              // everything but the tree
+    void* tree = nullptr;               // nodes, then leaf-ordered triangles
+    uint64_t tree_tris = 0;             // byte offset of the triangles
     ReinaSceneInfo info{};
-    std::vector<rt::Bvh8Node> host_nodes;   // kept for export
-    std::vector<rt::QBvh8Node> host_qnodes; // quantized copy (REINA_RT_NODES_QUANTIZED)
     bool quantized = false;
-    float device_build_ms = 0.0f;       // GPU time of a REINA_RT_BUILD_DEVICE build
-    std::vector<float> host_tris;
     // light-sampling tables (next-event estimation)
     std::vector<rt::EmissiveInst> emi;
     std::vector<float> tri_cdf;

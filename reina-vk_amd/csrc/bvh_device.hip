@@ -37,6 +37,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -65,6 +66,7 @@ struct Box6 {   // ordered-integer keys: lo (min), hi (max)
 // scene box (b) and centroid bounds (c)
 struct SceneBounds {
     Box6 b, c;
+    uint32_t nonfinite;   // k_flatten: some coordinate is infinite or NaN
 };
 
 __device__ __forceinline__ void tri_box(const float* w, float* lo, float* hi) {
@@ -94,6 +96,44 @@ __device__ __forceinline__ float wave_max(float v) {
 // adding its bounds with 12 atomics: one set per wave (61,000 atomics on 12
 // words for 327,686 triangles) took 700 us.
 constexpr uint32_t kPrepBlocks = 512;
+// World-space triangles, world = ((c0 x + c1 y) + c2 z) + c3 in the host
+// flattening's operation order, and the instance and primitive of every
+// triangle; w may be null (only the ids). A thread finds its instance by
+// bisection over the first-triangle ids (an instance without triangles shares
+// its successor's id and is never the last one at or below g). It reads and
+// writes ~100 bytes per triangle once: 14 us for 327,686 triangles, where the
+// loop on the host and the upload of its result took 2.6 ms.
+__global__ __launch_bounds__(256) void k_flatten(const InstanceRec* __restrict__ inst, uint32_t num_inst,
+                                                 const float4* __restrict__ vertices,
+                                                 const uint32_t* __restrict__ indices, uint32_t n,
+                                                 float* __restrict__ w, uint32_t* __restrict__ tri_inst,
+                                                 uint32_t* __restrict__ tri_prim, SceneBounds* sb) {
+    const uint32_t g = blockIdx.x * 256u + threadIdx.x;
+    if (g >= n) return;
+    uint32_t a = 0, b = num_inst;   // inst[a].tri_base <= g; inst[b].tri_base > g
+    while (b - a > 1) {
+        const uint32_t m = (a + b) / 2;
+        if (inst[m].tri_base <= g) a = m; else b = m;
+    }
+    const InstanceRec& r = inst[a];
+    const uint32_t prim = g - r.tri_base;
+    tri_inst[g] = a;
+    tri_prim[g] = prim;
+    if (!w) return;
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float4 v = vertices[indices[3ull * prim + r.index_offset + k]];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const float o = ((r.c0[c] * v.x + r.c1[c] * v.y) + r.c2[c] * v.z) + r.c3[c];
+            w[9ull * g + 3 * k + c] = o;
+            bad |= !(fabsf(o) < INFINITY);
+        }
+    }
+    if (bad) sb->nonfinite = 1;
+}
+
 __global__ __launch_bounds__(256) void k_prep(const float* __restrict__ wtri, uint32_t n, float4* __restrict__ plo,
                                               float4* __restrict__ phi, uint32_t* __restrict__ ref, SceneBounds* sb) {
     __shared__ float s_b[4][12];
@@ -1081,14 +1121,18 @@ __global__ void k_collapse_write(const BNode* __restrict__ nodes, const DpRec* _
     out[items[i].out] = nd;
 }
 
-template <typename T>
-struct DBuf {   // owns one device allocation; not copyable (a copy would free it twice)
-    T* p = nullptr;
-    DBuf() = default;
-    DBuf(const DBuf&) = delete;
-    DBuf& operator=(const DBuf&) = delete;
-    ~DBuf() { if (p) (void)hipFree(p); }
-    hipError_t alloc(size_t n) { return hipMalloc(&p, (n ? n : 1) * sizeof(T)); }
+// One device allocation for every buffer of a build: a hipMalloc and a hipFree
+// for each of the ~30 of them took 2.2 of a 327,686-triangle build's 14 ms.
+// take() is called in the same order twice, first with no base to add up the
+// bytes.
+struct Carver {
+    char* base = nullptr;
+    size_t bytes = 0;
+    template <typename T>
+    void take(T*& p, size_t n) {
+        p = reinterpret_cast<T*>(base + bytes);
+        bytes += ((n ? n : 1) * sizeof(T) + 255) & ~(size_t)255;
+    }
 };
 
 inline uint32_t blocks(uint64_t n, uint32_t b = 256) { return (uint32_t)((n + b - 1) / b); }
@@ -1168,24 +1212,18 @@ __global__ __launch_bounds__(1024) void k_scan_pair(const uint32_t* __restrict__
 // need at most 4 levels of 1024-element blocks).
 struct ScanTmp {
     static constexpr int kLevels = 4;
-    DBuf<uint32_t> lv[2 * kLevels];
-    hipError_t ensure(uint32_t n) {
+    uint32_t* lv[2 * kLevels] = {};
+    void carve(Carver& a, uint32_t n) {
         size_t k = 0;
         for (uint32_t m = n; m > kScanBlock; m = (m + kScanBlock - 1) / kScanBlock, ++k) {
             const uint32_t nb = (m + kScanBlock - 1) / kScanBlock;
-            if (k >= (size_t)kLevels) return hipErrorInvalidValue;
-            if (!lv[2 * k].p) {
-                hipError_t e = lv[2 * k].alloc(nb);
-                if (e != hipSuccess) return e;
-                e = lv[2 * k + 1].alloc(nb);
-                if (e != hipSuccess) return e;
-            }
+            a.take(lv[2 * k], nb);
+            a.take(lv[2 * k + 1], nb);
         }
-        return hipSuccess;
     }
 };
 
-// out[i] = in[0] + ... + in[i - 1]; tmp must have been sized for n by ensure().
+// out[i] = in[0] + ... + in[i - 1]; tmp must have been carved for n or more.
 hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint32_t n, ScanTmp& tmp, size_t level, hipStream_t st) {
     if (n == 0) return hipSuccess;
     const uint32_t nb = (n + kScanBlock - 1) / kScanBlock;
@@ -1193,8 +1231,8 @@ hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint32_t n, ScanTmp& tmp,
         hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(256), 0, st, in, out, n, nullptr);
         return hipGetLastError();
     }
-    uint32_t* sums = tmp.lv[2 * level].p;
-    uint32_t* offs = tmp.lv[2 * level + 1].p;
+    uint32_t* sums = tmp.lv[2 * level];
+    uint32_t* offs = tmp.lv[2 * level + 1];
     hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(256), 0, st, in, out, n, sums);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1203,6 +1241,93 @@ hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint32_t n, ScanTmp& tmp,
     hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(256), 0, st, out, n, offs);
     return hipGetLastError();
 }
+
+// Terms of bvh8_sah_cost, the sum over the nodes in FP64: each block's part in
+// part[block], the root's area in part[gridDim.x]. The blocks' parts are added
+// in order on the host, so the result does not depend on the schedule. 13 us
+// for 65,000 nodes (16 MB); bringing them to the host for it took 2.5 ms.
+__device__ __forceinline__ double area6(double lx, double ly, double lz, double hx, double hy, double hz) {
+    const double dx = hx - lx, dy = hy - ly, dz = hz - lz;
+    return 2.0 * (dx * dy + dy * dz + dz * dx);
+}
+
+constexpr uint32_t kSahBlocks = 256;
+
+__global__ __launch_bounds__(256) void k_sah(const Bvh8Node* __restrict__ nodes, uint32_t n, double* __restrict__ part) {
+    __shared__ double s_p[256];
+    double rl[3] = {INFINITY, INFINITY, INFINITY}, rh[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int k = 0; k < 8; ++k) {
+        if (!nodes[0].meta[k]) continue;
+        const double l[3] = {nodes[0].lo_x[k], nodes[0].lo_y[k], nodes[0].lo_z[k]};
+        const double h[3] = {nodes[0].hi_x[k], nodes[0].hi_y[k], nodes[0].hi_z[k]};
+        for (int a = 0; a < 3; ++a) { rl[a] = l[a] < rl[a] ? l[a] : rl[a]; rh[a] = rh[a] < h[a] ? h[a] : rh[a]; }
+    }
+    const double ra = area6(rl[0], rl[1], rl[2], rh[0], rh[1], rh[2]);
+    double sum = 0.0;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
+        const Bvh8Node& nd = nodes[i];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const uint8_t m = nd.meta[k];
+            if (!m) continue;
+            const double a = area6(nd.lo_x[k], nd.lo_y[k], nd.lo_z[k], nd.hi_x[k], nd.hi_y[k], nd.hi_z[k]) / ra;
+            sum += (m & 0x80) ? a : a * ((m >> 5) & 3);
+        }
+    }
+    s_p[threadIdx.x] = sum;
+    for (uint32_t d = 128; d > 0; d /= 2) {
+        __syncthreads();
+        if (threadIdx.x < d) s_p[threadIdx.x] += s_p[threadIdx.x + d];
+    }
+    if (threadIdx.x == 0) {
+        part[blockIdx.x] = s_p[0];
+        if (blockIdx.x == 0) part[gridDim.x] = ra;
+    }
+}
+
+struct BuildBufs {
+    float* w;
+    float4 *plo, *phi;
+    uint32_t *ref0, *ref1;
+    SceneBounds* sb;
+    BuildCtl* ctl;
+    BNode* nodes;
+    Task *t0, *t1, *b0, *b1;
+    BigState *s0, *s1;
+    uint32_t *ct0, *ct1, *cl;
+    SmallTask* small;
+    uint32_t *parent, *arrive;
+    DpRec* dp;
+    Bvh8Node* out;
+    float4* otri;
+    Item *it0, *it1;
+    uint32_t *ck, *ni, *nt, *si, *stri, *tot;
+    double* sah;
+    ScanTmp scan;
+    // sizes of the task lists and of the tree
+    uint32_t cap_large, cap_small, cap_big, cap_chunks, out_cap;
+
+    void carve(Carver& a, uint32_t n) {
+        cap_large = n / (kSmall + 1) + 2;
+        cap_small = n / 2 + 2;
+        cap_big = n / (kBig + 1) + 2;
+        cap_chunks = n / kChunk + cap_big + 2;
+        out_cap = std::max(1u, n - 1) + 1;
+        a.take(w, 9ull * n);
+        a.take(plo, n); a.take(phi, n); a.take(ref0, n); a.take(ref1, n);
+        a.take(sb, 1); a.take(ctl, 1); a.take(nodes, 2ull * n);
+        a.take(t0, cap_large); a.take(t1, cap_large); a.take(small, cap_small);
+        a.take(b0, cap_big); a.take(b1, cap_big); a.take(s0, cap_big); a.take(s1, cap_big);
+        a.take(ct0, cap_chunks); a.take(ct1, cap_chunks); a.take(cl, cap_chunks);
+        a.take(parent, 2ull * n); a.take(arrive, n); a.take(dp, n);
+        a.take(out, out_cap); a.take(otri, 3ull * n);
+        a.take(it0, out_cap); a.take(it1, out_cap);
+        a.take(ck, 8ull * out_cap); a.take(ni, out_cap + 1); a.take(nt, out_cap + 1);
+        a.take(si, out_cap + 1); a.take(stri, out_cap + 1); a.take(tot, 2);
+        a.take(sah, kSahBlocks + 1);
+        scan.carve(a, out_cap + 1);
+    }
+};
 
 }  // namespace
 
@@ -1215,52 +1340,69 @@ hipError_t scan_u32(const uint32_t* in, uint32_t* out, uint32_t n, ScanTmp& tmp,
         }                                                                         \
     } while (0)
 
-bool build_bvh8_device(const float* tri, uint64_t ntri, Bvh8Result& out, std::string& err, float* device_ms) {
-    out = Bvh8Result();
-    if (ntri >= (1ull << 24)) {
+hipError_t launch_triangle_ids(const DeviceMesh& m, hipStream_t st) {
+    if (m.num_tris == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_flatten, dim3(blocks(m.num_tris)), dim3(256), 0, st, m.inst, m.num_inst, m.vertices, m.indices,
+                       m.num_tris, (float*)nullptr, m.tri_inst, m.tri_prim, (SceneBounds*)nullptr);
+    return hipGetLastError();
+}
+
+DeviceBvh::~DeviceBvh() {
+    if (scratch) (void)hipFree(scratch);
+}
+
+bool build_bvh8_device(const DeviceMesh& mesh, const std::function<void(std::vector<float>&)>& flatten, DeviceBvh& out,
+                       std::string& err) {
+    const uint32_t n = mesh.num_tris;
+    if (n >= (1u << 24)) {
         err = "more than 2^24 triangles";
         return false;
-    }
-    const uint32_t n = (uint32_t)ntri;
-    if (n == 0) {   // one empty root node, as the host builder
-        out.nodes.resize(1);
-        std::memset(out.nodes.data(), 0, sizeof(Bvh8Node));
-        out.max_depth = 1;
-        return true;
     }
     hipStream_t st = nullptr;
     D_TRY(hipStreamCreate(&st));
     struct StreamGuard { hipStream_t s; ~StreamGuard() { (void)hipStreamDestroy(s); } } sg{st};
-    hipEvent_t e0, e1;
-    D_TRY(hipEventCreate(&e0));
-    D_TRY(hipEventCreate(&e1));
-    struct EvGuard { hipEvent_t a, b; ~EvGuard() { (void)hipEventDestroy(a); (void)hipEventDestroy(b); } } eg{e0, e1};
-    DBuf<float> d_w;
-    D_TRY(d_w.alloc(9ull * n));
-    D_TRY(hipMemcpyAsync(d_w.p, tri, 36ull * n, hipMemcpyHostToDevice, st));
-    D_TRY(hipEventRecord(e0, st));
-    DBuf<float4> d_plo, d_phi;
-    DBuf<uint32_t> d_ref0, d_ref1;
-    DBuf<SceneBounds> d_sb;
-    DBuf<BuildCtl> d_ctl;
-    DBuf<BNode> d_nodes;
-    D_TRY(d_plo.alloc(n)); D_TRY(d_phi.alloc(n)); D_TRY(d_ref0.alloc(n)); D_TRY(d_ref1.alloc(n));
-    D_TRY(d_sb.alloc(1)); D_TRY(d_ctl.alloc(1)); D_TRY(d_nodes.alloc(2ull * n));
-    {
-        SceneBounds init;
-        for (int a = 0; a < 3; ++a) {
-            init.b.lo[a] = init.c.lo[a] = 0xFFFFFFFFu;
-            init.b.hi[a] = init.c.hi[a] = 0u;
-        }
-        D_TRY(hipMemcpyAsync(d_sb.p, &init, sizeof init, hipMemcpyHostToDevice, st));
-        BuildCtl c{0u, 0u, 0u, 0u, 0u, kNone};
-        D_TRY(hipMemcpyAsync(d_ctl.p, &c, sizeof c, hipMemcpyHostToDevice, st));
+    if (n == 0) {   // one empty root node, as the host builder
+        Bvh8Node empty;
+        std::memset(&empty, 0, sizeof empty);
+        D_TRY(hipMalloc(&out.scratch, sizeof empty));
+        D_TRY(hipMemcpy(out.scratch, &empty, sizeof empty, hipMemcpyHostToDevice));
+        out.nodes = (const Bvh8Node*)out.scratch;
+        out.num_nodes = out.max_depth = 1;
+        return true;
     }
-    hipLaunchKernelGGL(k_prep, dim3(std::min(blocks(n), kPrepBlocks)), dim3(256), 0, st, d_w.p, n, d_plo.p, d_phi.p, d_ref0.p, d_sb.p);
-    D_TRY(hipGetLastError());
+    BuildBufs B;
+    Carver carver;
+    B.carve(carver, n);
+    D_TRY(hipMalloc(&out.scratch, carver.bytes));
+    carver = Carver{(char*)out.scratch, 0};
+    B.carve(carver, n);
     SceneBounds sb;
-    D_TRY(hipMemcpyAsync(&sb, d_sb.p, sizeof sb, hipMemcpyDeviceToHost, st));
-    D_TRY(hipStreamSynchronize(st));
+    for (int pass = 0;; ++pass) {
+        for (int a = 0; a < 3; ++a) {
+            sb.b.lo[a] = sb.c.lo[a] = 0xFFFFFFFFu;
+            sb.b.hi[a] = sb.c.hi[a] = 0u;
+        }
+        sb.nonfinite = 0;
+        D_TRY(hipMemcpyAsync(B.sb, &sb, sizeof sb, hipMemcpyHostToDevice, st));
+        if (pass == 0) {
+            BuildCtl c{0u, 0u, 0u, 0u, 0u, kNone};
+            D_TRY(hipMemcpyAsync(B.ctl, &c, sizeof c, hipMemcpyHostToDevice, st));
+            hipLaunchKernelGGL(k_flatten, dim3(blocks(n)), dim3(256), 0, st, mesh.inst, mesh.num_inst, mesh.vertices,
+                               mesh.indices, n, B.w, mesh.tri_inst, mesh.tri_prim, B.sb);
+            D_TRY(hipGetLastError());
+        }
+        hipLaunchKernelGGL(k_prep, dim3(std::min(blocks(n), kPrepBlocks)), dim3(256), 0, st, B.w, n, B.plo, B.phi, B.ref0, B.sb);
+        D_TRY(hipGetLastError());
+        D_TRY(hipMemcpyAsync(&sb, B.sb, sizeof sb, hipMemcpyDeviceToHost, st));
+        D_TRY(hipStreamSynchronize(st));
+        if (!sb.nonfinite) break;
+        // sign and payload of a NaN differ between the device's and the host's
+        // arithmetic and take part in the bounds' keys: such a scene keeps the
+        // host's coordinates
+        std::vector<float> w;
+        flatten(w);
+        D_TRY(hipMemcpy(B.w, w.data(), 36ull * n, hipMemcpyHostToDevice));
+    }
     auto unkey = [](uint32_t k) {
         const uint32_t u = (k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k;
         float f;
@@ -1268,17 +1410,6 @@ bool build_bvh8_device(const float* tri, uint64_t ntri, Bvh8Result& out, std::st
         return f;
     };
     // binary build: levels of large tasks, then every small task
-    const uint32_t cap_large = n / (kSmall + 1) + 2;
-    const uint32_t cap_small = n / 2 + 2;
-    const uint32_t cap_big = n / (kBig + 1) + 2;
-    const uint32_t cap_chunks = n / kChunk + cap_big + 2;
-    DBuf<Task> d_t0, d_t1, d_b0, d_b1;
-    DBuf<BigState> d_s0, d_s1;
-    DBuf<uint32_t> d_ct0, d_ct1, d_cl;
-    DBuf<SmallTask> d_small;
-    D_TRY(d_t0.alloc(cap_large)); D_TRY(d_t1.alloc(cap_large)); D_TRY(d_small.alloc(cap_small));
-    D_TRY(d_b0.alloc(cap_big)); D_TRY(d_b1.alloc(cap_big)); D_TRY(d_s0.alloc(cap_big)); D_TRY(d_s1.alloc(cap_big));
-    D_TRY(d_ct0.alloc(cap_chunks)); D_TRY(d_ct1.alloc(cap_chunks)); D_TRY(d_cl.alloc(cap_chunks));
     uint32_t root = kNone;
     uint32_t n_small = 0;
     if (n == 1) {
@@ -1291,10 +1422,10 @@ bool build_bvh8_device(const float* tri, uint64_t ntri, Bvh8Result& out, std::st
         b.tri = 0;
         b.lo[0] = lo.x; b.lo[1] = lo.y; b.lo[2] = lo.z;
         b.hi[0] = hi.x; b.hi[1] = hi.y; b.hi[2] = hi.z;
-        D_TRY(hipMemcpyAsync(d_nodes.p, &b, sizeof b, hipMemcpyHostToDevice, st));
+        D_TRY(hipMemcpyAsync(B.nodes, &b, sizeof b, hipMemcpyHostToDevice, st));
     } else if (n <= kSmall) {
         SmallTask t{0u, n, kNone, 0u};
-        D_TRY(hipMemcpyAsync(d_small.p, &t, sizeof t, hipMemcpyHostToDevice, st));
+        D_TRY(hipMemcpyAsync(B.small, &t, sizeof t, hipMemcpyHostToDevice, st));
         n_small = 1;
     } else {
         Task t;
@@ -1306,9 +1437,9 @@ bool build_bvh8_device(const float* tri, uint64_t ntri, Bvh8Result& out, std::st
             t.clo[a] = unkey(sb.c.lo[a]); t.chi[a] = unkey(sb.c.hi[a]);
         }
         uint32_t ntasks = n > kBig ? 0 : 1, nbig = n > kBig ? 1 : 0, nchunks = n > kBig ? t.nchunks : 0, levels = 0;
-        Task *cur = d_t0.p, *nxt = d_t1.p, *bcur = d_b0.p, *bnxt = d_b1.p;
-        BigState *scur = d_s0.p, *snxt = d_s1.p;
-        uint32_t *ccur = d_ct0.p, *cnxt = d_ct1.p;
+        Task *cur = B.t0, *nxt = B.t1, *bcur = B.b0, *bnxt = B.b1;
+        BigState *scur = B.s0, *snxt = B.s1;
+        uint32_t *ccur = B.ct0, *cnxt = B.ct1;
         D_TRY(hipMemcpyAsync(nbig ? bcur : cur, &t, sizeof t, hipMemcpyHostToDevice, st));
         if (nbig) {
             hipLaunchKernelGGL(k_big_root, dim3(1), dim3(256), 0, st, bcur, scur, ccur);
@@ -1319,32 +1450,32 @@ bool build_bvh8_device(const float* tri, uint64_t ntri, Bvh8Result& out, std::st
                 err = "device BVH build did not converge";
                 return false;
             }
-            D_TRY(hipMemsetAsync(&d_ctl.p->n_next, 0, 12, st));   // n_next, n_big, n_chunks
+            D_TRY(hipMemsetAsync(&B.ctl->n_next, 0, 12, st));   // n_next, n_big, n_chunks
             if (nbig) {
-                hipLaunchKernelGGL(k_big_bin, dim3(nchunks), dim3(256), 0, st, bcur, ccur, d_plo.p, d_phi.p, d_ref0.p,
-                                   d_ref1.p, scur);
+                hipLaunchKernelGGL(k_big_bin, dim3(nchunks), dim3(256), 0, st, bcur, ccur, B.plo, B.phi, B.ref0,
+                                   B.ref1, scur);
                 D_TRY(hipGetLastError());
                 hipLaunchKernelGGL(k_big_plan, dim3(nbig), dim3(256), 0, st, bcur, scur);
                 D_TRY(hipGetLastError());
-                hipLaunchKernelGGL(k_big_count, dim3(nchunks), dim3(256), 0, st, bcur, ccur, d_plo.p, d_phi.p, d_ref0.p,
-                                   d_ref1.p, scur, d_cl.p);
+                hipLaunchKernelGGL(k_big_count, dim3(nchunks), dim3(256), 0, st, bcur, ccur, B.plo, B.phi, B.ref0,
+                                   B.ref1, scur, B.cl);
                 D_TRY(hipGetLastError());
-                hipLaunchKernelGGL(k_big_partition, dim3(nchunks), dim3(256), 0, st, bcur, ccur, d_plo.p, d_phi.p,
-                                   d_ref0.p, d_ref1.p, scur, d_cl.p, d_nodes.p);
+                hipLaunchKernelGGL(k_big_partition, dim3(nchunks), dim3(256), 0, st, bcur, ccur, B.plo, B.phi,
+                                   B.ref0, B.ref1, scur, B.cl, B.nodes);
                 D_TRY(hipGetLastError());
-                hipLaunchKernelGGL(k_big_emit, dim3(nbig), dim3(256), 0, st, bcur, scur, n, d_nodes.p, nxt, bnxt, snxt,
-                                   cnxt, d_small.p, d_ctl.p);
+                hipLaunchKernelGGL(k_big_emit, dim3(nbig), dim3(256), 0, st, bcur, scur, n, B.nodes, nxt, bnxt, snxt,
+                                   cnxt, B.small, B.ctl);
                 D_TRY(hipGetLastError());
             }
             if (ntasks) {
-                hipLaunchKernelGGL(k_split_tasks, dim3(ntasks), dim3(256), 0, st, cur, n, d_plo.p, d_phi.p, d_ref0.p,
-                                   d_ref1.p, d_nodes.p, nxt, d_small.p, d_ctl.p);
+                hipLaunchKernelGGL(k_split_tasks, dim3(ntasks), dim3(256), 0, st, cur, n, B.plo, B.phi, B.ref0,
+                                   B.ref1, B.nodes, nxt, B.small, B.ctl);
                 D_TRY(hipGetLastError());
             }
             BuildCtl c;
-            D_TRY(hipMemcpyAsync(&c, d_ctl.p, sizeof c, hipMemcpyDeviceToHost, st));
+            D_TRY(hipMemcpyAsync(&c, B.ctl, sizeof c, hipMemcpyDeviceToHost, st));
             D_TRY(hipStreamSynchronize(st));
-            if (c.n_next > cap_large || c.n_small > cap_small || c.n_big > cap_big || c.n_chunks > cap_chunks) {
+            if (c.n_next > B.cap_large || c.n_small > B.cap_small || c.n_big > B.cap_big || c.n_chunks > B.cap_chunks) {
                 err = "device BVH build task list overflow";
                 return false;
             }
@@ -1359,13 +1490,13 @@ bool build_bvh8_device(const float* tri, uint64_t ntri, Bvh8Result& out, std::st
         }
     }
     if (n_small) {
-        hipLaunchKernelGGL(k_small_tasks, dim3((n_small + 3) / 4), dim3(256), 0, st, d_small.p, n_small, n, d_plo.p,
-                           d_phi.p, d_ref0.p, d_ref1.p, d_nodes.p, d_ctl.p);
+        hipLaunchKernelGGL(k_small_tasks, dim3((n_small + 3) / 4), dim3(256), 0, st, B.small, n_small, n, B.plo,
+                           B.phi, B.ref0, B.ref1, B.nodes, B.ctl);
         D_TRY(hipGetLastError());
     }
     if (n > 1) {
         BuildCtl c;
-        D_TRY(hipMemcpyAsync(&c, d_ctl.p, sizeof c, hipMemcpyDeviceToHost, st));
+        D_TRY(hipMemcpyAsync(&c, B.ctl, sizeof c, hipMemcpyDeviceToHost, st));
         D_TRY(hipStreamSynchronize(st));
         root = c.root;
         if (root < n || root >= 2 * n - 1) {
@@ -1374,74 +1505,57 @@ bool build_bvh8_device(const float* tri, uint64_t ntri, Bvh8Result& out, std::st
         }
     }
     // collapse: the SAH-optimal slot distribution of every binary node, bottom-up
-    DBuf<uint32_t> d_parent, d_arrive;
-    DBuf<DpRec> d_dp;
-    D_TRY(d_parent.alloc(2ull * n)); D_TRY(d_arrive.alloc(n)); D_TRY(d_dp.alloc(n));
-    D_TRY(hipMemsetAsync(d_parent.p, 0xFF, sizeof(uint32_t) * (2ull * n), st));
+    D_TRY(hipMemsetAsync(B.parent, 0xFF, sizeof(uint32_t) * (2ull * n), st));
     if (n > 1) {
-        hipLaunchKernelGGL(k_parents, dim3(blocks(n - 1)), dim3(256), 0, st, d_nodes.p, n, d_parent.p, d_arrive.p);
+        hipLaunchKernelGGL(k_parents, dim3(blocks(n - 1)), dim3(256), 0, st, B.nodes, n, B.parent, B.arrive);
         D_TRY(hipGetLastError());
         if (n_small) {
-            hipLaunchKernelGGL(k_collapse_dp_small, dim3((n_small + 3) / 4), dim3(256), 0, st, d_small.p, n_small, n,
-                               d_nodes.p, d_dp.p);
+            hipLaunchKernelGGL(k_collapse_dp_small, dim3((n_small + 3) / 4), dim3(256), 0, st, B.small, n_small, n,
+                               B.nodes, B.dp);
             D_TRY(hipGetLastError());
         }
-        hipLaunchKernelGGL(k_collapse_dp, dim3(blocks((uint64_t)n + n_small)), dim3(256), 0, st, d_nodes.p, n, d_small.p,
-                           n_small, d_parent.p, d_arrive.p, d_dp.p);
+        hipLaunchKernelGGL(k_collapse_dp, dim3(blocks((uint64_t)n + n_small)), dim3(256), 0, st, B.nodes, n, B.small,
+                           n_small, B.parent, B.arrive, B.dp);
         D_TRY(hipGetLastError());
     }
-    const uint32_t n_internal = n - 1;
-    DBuf<Bvh8Node> d_out;
-    DBuf<float4> d_otri;
-    DBuf<Item> d_it0, d_it1;
-    DBuf<uint32_t> d_ck, d_ni, d_nt, d_si, d_stri, d_tot;
-    D_TRY(d_tot.alloc(2));
-    const uint32_t out_cap = std::max(1u, n_internal) + 1;
-    D_TRY(d_out.alloc(out_cap)); D_TRY(d_otri.alloc(3ull * n));
-    D_TRY(d_it0.alloc(out_cap)); D_TRY(d_it1.alloc(out_cap));
-    D_TRY(d_ck.alloc(8ull * out_cap)); D_TRY(d_ni.alloc(out_cap + 1)); D_TRY(d_nt.alloc(out_cap + 1));
-    D_TRY(d_si.alloc(out_cap + 1)); D_TRY(d_stri.alloc(out_cap + 1));
-    ScanTmp scan_tmp;
-    D_TRY(scan_tmp.ensure(out_cap + 1));
     {
         Item r0{root, 0};
-        D_TRY(hipMemcpyAsync(d_it0.p, &r0, sizeof r0, hipMemcpyHostToDevice, st));
+        D_TRY(hipMemcpyAsync(B.it0, &r0, sizeof r0, hipMemcpyHostToDevice, st));
     }
     uint32_t nitems = 1, out_nodes = 1, out_tris = 0, depth = 0;
-    Item* items = d_it0.p;
-    Item* nitems_buf = d_it1.p;
+    Item* items = B.it0;
+    Item* nitems_buf = B.it1;
     while (nitems > 0) {
         depth++;
-        hipLaunchKernelGGL(k_collapse_count, dim3(blocks(nitems, 64)), dim3(64), 0, st, d_nodes.p, d_dp.p, n, items,
-                           nitems, d_ck.p, d_ni.p, d_nt.p);
+        hipLaunchKernelGGL(k_collapse_count, dim3(blocks(nitems, 64)), dim3(64), 0, st, B.nodes, B.dp, n, items,
+                           nitems, B.ck, B.ni, B.nt);
         D_TRY(hipGetLastError());
         uint32_t tot[2] = {0, 0};
         if (nitems <= kScanSmall) {
-            hipLaunchKernelGGL(k_scan_pair, dim3(1), dim3(1024), 0, st, d_ni.p, d_nt.p, d_si.p, d_stri.p, nitems, d_tot.p);
+            hipLaunchKernelGGL(k_scan_pair, dim3(1), dim3(1024), 0, st, B.ni, B.nt, B.si, B.stri, nitems, B.tot);
             D_TRY(hipGetLastError());
-            D_TRY(hipMemcpyAsync(tot, d_tot.p, sizeof tot, hipMemcpyDeviceToHost, st));
+            D_TRY(hipMemcpyAsync(tot, B.tot, sizeof tot, hipMemcpyDeviceToHost, st));
         } else {
-            D_TRY(hipMemsetAsync(d_ni.p + nitems, 0, 4, st));
-            D_TRY(hipMemsetAsync(d_nt.p + nitems, 0, 4, st));
-            D_TRY(scan_u32(d_ni.p, d_si.p, nitems + 1, scan_tmp, 0, st));
-            D_TRY(scan_u32(d_nt.p, d_stri.p, nitems + 1, scan_tmp, 0, st));
-            D_TRY(hipMemcpyAsync(&tot[0], d_si.p + nitems, 4, hipMemcpyDeviceToHost, st));
-            D_TRY(hipMemcpyAsync(&tot[1], d_stri.p + nitems, 4, hipMemcpyDeviceToHost, st));
+            D_TRY(hipMemsetAsync(B.ni + nitems, 0, 4, st));
+            D_TRY(hipMemsetAsync(B.nt + nitems, 0, 4, st));
+            D_TRY(scan_u32(B.ni, B.si, nitems + 1, B.scan, 0, st));
+            D_TRY(scan_u32(B.nt, B.stri, nitems + 1, B.scan, 0, st));
+            D_TRY(hipMemcpyAsync(&tot[0], B.si + nitems, 4, hipMemcpyDeviceToHost, st));
+            D_TRY(hipMemcpyAsync(&tot[1], B.stri + nitems, 4, hipMemcpyDeviceToHost, st));
         }
         D_TRY(hipStreamSynchronize(st));
-        if (out_nodes + tot[0] > out_cap || out_tris + tot[1] > n) {
+        if (out_nodes + tot[0] > B.out_cap || out_tris + tot[1] > n) {
             err = "device BVH collapse overflow";
             return false;
         }
-        hipLaunchKernelGGL(k_collapse_write, dim3(blocks(nitems, 64)), dim3(64), 0, st, d_nodes.p, d_dp.p, n, items,
-                           nitems, d_ck.p, d_si.p, d_stri.p, out_nodes, out_tris, d_w.p, d_out.p, d_otri.p, nitems_buf);
+        hipLaunchKernelGGL(k_collapse_write, dim3(blocks(nitems, 64)), dim3(64), 0, st, B.nodes, B.dp, n, items,
+                           nitems, B.ck, B.si, B.stri, out_nodes, out_tris, B.w, B.out, B.otri, nitems_buf);
         D_TRY(hipGetLastError());
         out_nodes += tot[0];
         out_tris += tot[1];
         nitems = tot[0];
         std::swap(items, nitems_buf);
     }
-    D_TRY(hipEventRecord(e1, st));
     if (out_tris != n) {
         err = "device BVH lost triangles";
         return false;
@@ -1450,16 +1564,21 @@ bool build_bvh8_device(const float* tri, uint64_t ntri, Bvh8Result& out, std::st
         err = "too many BVH8 nodes for the index encoding (max 2^24)";
         return false;
     }
-    out.nodes.resize(out_nodes);
-    out.tris.resize(12ull * n);
-    D_TRY(hipMemcpyAsync(out.nodes.data(), d_out.p, sizeof(Bvh8Node) * out_nodes, hipMemcpyDeviceToHost, st));
-    D_TRY(hipMemcpyAsync(out.tris.data(), d_otri.p, 48ull * n, hipMemcpyDeviceToHost, st));
+    const uint32_t sah_blocks = std::min(blocks(out_nodes), kSahBlocks);
+    hipLaunchKernelGGL(k_sah, dim3(sah_blocks), dim3(256), 0, st, B.out, out_nodes, B.sah);
+    D_TRY(hipGetLastError());
+    double part[kSahBlocks + 1];
+    D_TRY(hipMemcpyAsync(part, B.sah, sizeof(double) * (sah_blocks + 1), hipMemcpyDeviceToHost, st));
     D_TRY(hipStreamSynchronize(st));
-    float ms = 0.0f;
-    D_TRY(hipEventElapsedTime(&ms, e0, e1));
-    if (device_ms) *device_ms = ms;
+    if (part[sah_blocks] > 0.0) {
+        double sah = 1.0;   // the root node itself
+        for (uint32_t i = 0; i < sah_blocks; ++i) sah += part[i];
+        out.sah_cost = (float)sah;
+    }
+    out.nodes = B.out;
+    out.tris = B.otri;
+    out.num_nodes = out_nodes;
     out.max_depth = depth;
-    out.sah_cost = bvh8_sah_cost(out.nodes);
     return true;
 }
 

@@ -87,7 +87,8 @@ struct alignas(16) InstanceRec {
     uint32_t model;
     uint32_t tri_base;                  // first flattened triangle id
     float n0[3], n1[3], n2[3];          // columns of the inverse transpose of (c0, c1, c2)
-    float pad[3];
+    uint32_t index_offset;              // of the model's vertex indices
+    float pad[2];
 };
 static_assert(sizeof(InstanceRec) == 112, "instance record size");
 

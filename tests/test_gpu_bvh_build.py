@@ -88,3 +88,55 @@ def test_device_build_sizes(cuda, n, kind):
     assert torch.equal(ha.view(torch.int32), hb.view(torch.int32))
     a.close()
     b.close()
+
+
+def _flatten(arrays):
+    """world = ((c0 x + c1 y) + c2 z) + c3 in float32, instance by instance."""
+    out = []
+    v, idx = arrays["vertices"].reshape(-1, 4), arrays["indices"]
+    for i in arrays["instances"]:
+        m = arrays["models"][i["modelID"]]
+        c = i["transform"].astype(np.float32).reshape(4, 4)[:, :3]
+        first = int(m["indexOffset"])
+        p = v[idx[first:first + 3 * int(m["indexCount"])]][:, :3]
+        with np.errstate(invalid="ignore", over="ignore"):
+            out.append(((c[0] * p[:, :1] + c[1] * p[:, 1:2]) + c[2] * p[:, 2:3]) + c[3])
+    return np.concatenate(out).astype(np.float32).reshape(-1, 9)
+
+
+@pytest.mark.parametrize("flags", [0, abi.NODES_QUANTIZED, abi.BUILD_HOST])
+@pytest.mark.parametrize("sizes", [(1,), (3, 300, 1, 255), (64, 0, 1, 0), (0, 5000)])
+def test_world_triangles_are_the_host_arithmetic(cuda, sizes, flags):
+    """Triangles flattened on the device are, bit for bit, the float32
+    arithmetic above, also beside instances without triangles."""
+    rng = np.random.default_rng(len(sizes) * 100 + sum(sizes))
+    s = Scene()
+    for n in sizes:
+        v = np.concatenate([_soup(n, "soup").reshape(-1, 3), np.ones((3 * n, 1))], 1).astype(np.float32)
+        idx = rng.permutation(3 * n).astype(np.uint32)
+        md = ModelData(v, idx, np.tile(np.eye(3, dtype=np.float32), (3 * n, 1, 1)), idx.copy())
+        m = np.eye(4)
+        m[:3] = rng.normal(size=(3, 4))
+        s.add_object(md, m, Material(materialIdx=0))
+    a = s.build_arrays()
+    dev = reina_rt.DeviceScene(a, flags=flags)
+    t = dev.export_bvh()[1].reshape(-1, 3, 4)
+    got = np.empty((len(t), 9), np.float32)
+    got[t[:, 0, 3].copy().view(np.uint32)] = t[:, :, :3].reshape(-1, 9)
+    assert np.array_equal(got.view(np.uint32), _flatten(a).view(np.uint32))
+    dev.close()
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3.0e38])
+def test_non_finite_triangle_keeps_the_host_bits(cuda, value):
+    tri = np.array([[[0, 0, 0], [1, value, 0], [0, 1, 0]]], np.float32)
+    a = _arrays(tri)
+    a["instances"][0]["transform"][4] = 2.0    # x += 2 y overflows at 3e38
+    got = []
+    for flags in (0, abi.BUILD_HOST):
+        dev = reina_rt.DeviceScene(a, flags=flags)
+        got.append(dev.export_bvh()[1].reshape(3, 4)[:, :3].reshape(1, 9).copy())
+        dev.close()
+    assert not np.isfinite(got[0]).all()
+    assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    assert np.array_equal(got[0], _flatten(a), equal_nan=True)
