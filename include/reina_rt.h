@@ -355,7 +355,9 @@ typedef struct ReinaTuning {
     uint32_t shade_blocks;  /* shade blocks (256 threads), a multiple of 8                      */
     uint32_t waves_per_simd;/* traversal register budget: 0 (compiler's choice), 4, 5, 6 or 8      */
     uint32_t tail_paths;    /* when at most this many paths are live, the frame ends in one
-                               tail launch (per-wave extend/shade steps); 0 = never            */
+                               tail launch (per-wave extend/shade steps); 0 = never; the
+                               default, 2^20, stands for 2^22 in a trace without next-event
+                               estimation, COUNT or TIME_EXTEND                                */
     uint32_t claim_rays;    /* rays a traversal wave claims from its queue partition with one
                                atomic: 64, 128, 256 or 512 (0 = 128)                           */
 } ReinaTuning;

@@ -630,9 +630,11 @@ int reina_rt_trace(ReinaScene* s, const RtPushConsts* pc, float* image, uint32_t
     const uint32_t K = 4;   // iterations between queue-length readbacks
     s->tail_count = 0;
     s->xev_used = 0;
+    const uint32_t tail_paths = s->tune.tail_paths == kDefaultTailPaths && !nee && !timex && !count
+                                    ? kDefaultTailPathsPlain : s->tune.tail_paths;
     while (it < max_iters && live != 0) {
         const uint32_t slot = it % 3, in_q = it & 1u;
-        if (live <= s->tune.tail_paths) {
+        if (live <= tail_paths) {
             // few paths left: finish them in one launch
             HIP_TRY(hipEventRecord(s->tev0, st));
             HIP_TRY(launch_tail(s->sv, P, s->S, s->Q, in_q, s->ctrl, slot, s->stats, s->tune, (uint32_t)live, st));

@@ -27,6 +27,21 @@ int fail(int code, const std::string& msg);
 // Live paths at or below which reina_rt_trace ends the frame in one tail
 // launch (ReinaTuning.tail_paths default).
 constexpr uint32_t kDefaultTailPaths = 1u << 20;
+// What the default stands for in a trace without next-event estimation (and
+// without the options that count or time the extend kernel, which then has to
+// run): a frame of up to 2^22 paths is one tail launch from its first ray on.
+// The tail keeps a pixel's state and ray in registers, where a bounce
+// iteration moves ~200 bytes per ray through HBM and ends with its slowest
+// waves. ms at 2^20 | 2^22 | 2^24: 1080p 64 spp, 327,686 triangles
+// 88.8 | 72.8 | 72.3; 1080x1350 8.30 | 7.57 | 7.48; 1080p 2 spp, 1.05M
+// instanced triangles 2.20 | 1.33 | 1.28, 40 triangles 1.98 | 1.55 | 1.55.
+// Above, frames start as bounce iterations: 3840x2160 8 spp, 500,000 triangles
+// 29.4 | 28.7 | 30.5, instanced 14.6 | 14.3 | 14.7, 40 triangles
+// 27.4 | 25.6 | 20.7; 1080p in 8 sample groups 7.60 | 7.55 | 8.52. With
+// next-event estimation the tail's lockstep steps lose as often as they win
+// (1080p 8 spp at 2^20 | 2^22: icosphere 23.8 | 29.0, lobes 26.8 | 28.4,
+// textured 30.5 | 26.3).
+constexpr uint32_t kDefaultTailPathsPlain = 1u << 22;
 
 // Kernel parameters of one vkCmdTraceRaysKHR-equivalent render.
 inline TraceParams make_trace_params(const RtPushConsts* pc, uint32_t W, uint32_t H) {
