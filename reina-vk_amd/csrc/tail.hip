@@ -15,9 +15,9 @@
 // a lane holds it (loading and storing it around every shading cost 4-5% where
 // few waves hide the latency: 256x256 Cornell box 1533 -> 1462 us, 12 server
 // requests 26.2 -> 25.0 ms, 720p instanced 5448 -> 5301 us), and the wave does
-// not wait for its slowest
-// traversal: it keeps visiting nodes until `shade_min` lanes (or all
-// lanes holding a pixel, if fewer) have finished their traversal, shades
+// not wait for its slowest traversal: it keeps visiting nodes until enough
+// lanes (`shade_min`, or all lanes holding a pixel, if fewer; more while every
+// lane holds one) have finished their traversal, shades
 // those lanes only, and resumes the others where they stopped. A suspended
 // lane keeps its ray (ra, rb), closest hit and stack position; its slab
 // constants are recomputed from the ray when traversal resumes, so they are
@@ -86,6 +86,16 @@ __device__ __forceinline__ uint32_t tail_claim(Ctrl* ctrl, uint32_t slot, uint32
 // VGPRs, a few bytes more scratch than the compiler's own 188 VGPRs at 2
 // waves; the 1080p frame measured 2.6% faster); the NEE build keeps the
 // compiler's choice (at 168 VGPRs it would spill ~200 bytes per lane).
+//
+// Ready lanes that trigger shading (without NEE): shade_min while the wave has
+// empty lanes. A wave with a pixel in every lane waits for 3/8 more where more
+// blocks wait than the GPU holds (3 on each of 256 CUs): 1080p 64 spp at 32,
+// 40, 44, 48, 56 lanes 72.8, 70.8, 70.3, 70.3, 74.4 ms, 1080x1350 7.61, 7.50,
+// 7.38, 7.37, 7.62 ms. With fewer blocks no other wave fills the wait (256x256
+// 1.47 ms at 32, 1.49 at 44), nor in the server's mixed queue (12 requests
+// 24.8 and 25.1 ms).
+constexpr uint32_t kTailResidentBlocks = 3u * 256u;
+
 template <int SD, bool Q, bool NEE, bool MULTI>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NEE ? 0 : 3))) void k_tail(SceneView sv, TraceParams P, PathState S, Queues Q_, uint32_t in_q,
                                               Ctrl* ctrl, uint32_t slot, unsigned long long* stats,
@@ -102,6 +112,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NEE ? 0 : 3
     const void* nodes = Q ? static_cast<const void*>(sv.qnodes) : static_cast<const void*>(sv.nodes);
     const float4* tris = sv.tris;
     uint64_t num_nodes = sv.num_nodes;
+    const uint32_t shade_full = !MULTI && gridDim.x > kTailResidentBlocks ? min(64u, shade_min + 3u * shade_min / 8u)
+                                                                          : min(64u, shade_min);
     float4 ra = make_float4(0.0f, 0.0f, 0.0f, 0.0f), rb = ra;
     uint32_t nrays = 0, nshadow = 0, dummy_v = 0, dummy_t = 0;
     if constexpr (!NEE) {
@@ -151,7 +163,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NEE ? 0 : 3
                     nrays++;
                 }
                 const uint32_t held = (uint32_t)__popcll(holding);
-                uint32_t need = shade_min < held ? shade_min : held;
+                uint32_t need = held == 64u ? shade_full : min(shade_min, held);
                 if (need == 0u) need = 1u;   // every round shades at least one lane
                 for (;;) {
                     if (__ballot(tracing) == 0ull) break;
