@@ -376,9 +376,10 @@ int reina_rt_intersect(ReinaScene* scene, const ReinaRay* rays, ReinaHit* hits,
  * under HIP graph capture and tight serving loops. The traversal kernel's
  * claim counters and used-up flag (1152 bytes) live in a static device
  * array of the library, one per GPU, held until the process ends, and are zeroed by a fill kernel on
- * `stream` at every call. At most 2^30 rays per call (REINA_RT_ERR_INVALID_ARG
- * beyond). Calls that overlap on one GPU (different streams or threads) race
- * on the shared counters; serialise them. Hits equal reina_rt_intersect's. */
+ * `stream` at every call with more than 2^18 rays (fewer take one launch
+ * that needs neither). At most 2^30 rays per call (REINA_RT_ERR_INVALID_ARG
+ * beyond). Calls of more than 2^18 rays that overlap on one GPU (different streams
+ * or threads) race on the shared counters; serialise them. Hits equal reina_rt_intersect's. */
 int reina_rt_intersect_noalloc(ReinaScene* scene, const ReinaRay* rays, ReinaHit* hits, uint32_t n, void* stream);
 
 /* Bloom (blurX with threshold, blurY, combine) then ACES-fitted tone map to
