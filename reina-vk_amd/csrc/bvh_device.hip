@@ -790,6 +790,9 @@ __global__ __launch_bounds__(256) void k_small_tasks(const SmallTask* __restrict
         id = nid;
         lo = nlo;
         hi = nhi;
+        // no split has a finite cost (a box area overflows or is not a number): halve by
+        // position, as the larger tasks do; one triangle at a time would nest 63 deep
+        if (!(best < (double)INFINITY)) best_k = sz / 2u - 1u;
         const uint32_t nl = best_k + 1u, nr = sz - nl;
         const uint32_t node = n + T.begin + r0 + nl - 1u;
         if (nl == 1u && lane == r0) write_leaf(nodes, T.begin + r0, id, lo, hi);
@@ -880,7 +883,7 @@ __device__ __forceinline__ DpRec dp_node(const BNode& b, const float (&cl)[8], c
     const float A = area_f(b);
     const float cint = A * kCollapseNodeCost + dist[7];
     const float cleaf = b.count <= kLeafMax ? A * kCollapseTriCost * (float)b.count : INFINITY;
-    r.leaf = cleaf <= cint ? 1 : 0;
+    r.leaf = b.count <= kLeafMax && cleaf <= cint ? 1 : 0;   // cint, too, is infinite where an area overflows
     r.split8 = dk[7];
     r.pad0 = r.pad1 = 0;
     r.c[0] = fminf(cleaf, cint);

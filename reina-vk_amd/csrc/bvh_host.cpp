@@ -311,7 +311,8 @@ bool build_bvh8_host(const float* tri, uint64_t ntri, Bvh8Result& out, std::stri
             }
             const float cint = A * cN + dist[7];
             const float cleaf = sub_cnt[n] <= kMaxLeafTris ? A * cP * (float)sub_cnt[n] : INFINITY;
-            as_leaf[n] = cleaf <= cint ? 1 : 0;
+            // cint, too, is infinite where an area overflows
+            as_leaf[n] = sub_cnt[n] <= kMaxLeafTris && cleaf <= cint ? 1 : 0;
             c[0] = std::min(cleaf, cint);
             dk[(size_t)n * 8] = 0;
             for (int j = 2; j <= 8; ++j) {

@@ -140,3 +140,57 @@ def test_non_finite_triangle_keeps_the_host_bits(cuda, value):
     assert not np.isfinite(got[0]).all()
     assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
     assert np.array_equal(got[0], _flatten(a), equal_nan=True)
+
+
+def _same_hits(torch, a, b, rays):
+    h = [torch.zeros((len(rays), 4), device="cuda") for _ in range(2)]
+    for dev, out in zip((a, b), h):
+        dev.intersect(rays.data_ptr(), out.data_ptr(), len(rays))
+    torch.cuda.synchronize()
+    assert torch.equal(h[0].view(torch.int32), h[1].view(torch.int32))
+    return h[0]
+
+
+def _aimed_rays(torch, targets, seed, n=4096):
+    """Rays from around the unit cube to the targets, in turn."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    r = torch.zeros((n, 8), device="cuda")
+    r[:, 0:3] = torch.rand((n, 3), device="cuda", generator=g) * 5 - 0.5
+    c = torch.from_numpy(np.ascontiguousarray(targets, np.float32)).cuda()[torch.arange(n, device="cuda") % len(targets)]
+    r[:, 4:7] = torch.nn.functional.normalize(c - r[:, 0:3], dim=1)
+    r[:, 7] = 1e4
+    return r
+
+
+@pytest.mark.parametrize("n", [4, 64, 65, 5000])
+@pytest.mark.parametrize("scale", [1e19, 1e25, 1e37])
+def test_boxes_whose_area_overflows(cuda, n, scale):
+    """No split has a finite cost: leaves of 1..3 triangles all the same, every
+    triangle in one of them, and a depth that the traversal stack holds."""
+    torch = cuda
+    arrays = _arrays(_soup(n, "soup") * scale)
+    a, b = reina_rt.DeviceScene(arrays), reina_rt.DeviceScene(arrays, flags=abi.BUILD_HOST)
+    for dev in (a, b):
+        _check_tree(dev, n)
+        assert dev.info().max_depth <= 16
+    _same_hits(torch, a, b, _aimed_rays(torch, np.eye(3), n))
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("n", [4, 64, 65, 5000])
+@pytest.mark.parametrize("far", [1e20, 3e38])
+def test_one_huge_triangle_beside_others(cuda, n, far):
+    """A triangle whose box area overflows takes no other out of the tree."""
+    torch = cuda
+    t = _soup(n, "soup")
+    t[n // 3, 0] = (far, -far, far)
+    arrays = _arrays(t)
+    a, b = reina_rt.DeviceScene(arrays), reina_rt.DeviceScene(arrays, flags=abi.BUILD_HOST)
+    _check_tree(a, n)
+    _check_tree(b, n)
+    hits = _same_hits(torch, a, b, _aimed_rays(torch, t[np.arange(n) != n // 3].mean(1), n))
+    assert float((hits.view(torch.int32)[:, 1] >= 0).float().mean()) > 0.9
+    a.close()
+    b.close()

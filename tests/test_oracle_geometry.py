@@ -122,6 +122,42 @@ def check_bvh8_structure(nodes, tri_out, ntri):
     assert seen_nodes == set(range(N))
 
 
+def _leaf_counts(nodes):
+    m = nodes.reshape(-1, 256)[:, 200:208].astype(int)
+    return (m >> 5)[(m != 0) & (m < 0x80)]
+
+
+@pytest.mark.parametrize("scale", [1e19, 1e25, 1e37])
+@pytest.mark.parametrize("n", [4, 50, 500])
+def test_host_build_of_huge_coordinates(n, scale):
+    """Boxes whose area overflows: still leaves of 1..3 triangles and every
+    triangle in one of them."""
+    rng = np.random.default_rng(n)
+    t = ((rng.random((n, 1, 3)) * 4 + 0.1 * rng.normal(size=(n, 3, 3))) * scale).astype(np.float32).reshape(-1, 9)
+    nodes, tris, depth = reina_rt.bvh_build_host(t)
+    check_bvh8_structure(nodes, tris, n)
+    assert _leaf_counts(nodes).sum() == n and depth <= 17
+
+
+@pytest.mark.parametrize("far", [1e20, 3e38, np.inf, -np.inf])
+@pytest.mark.parametrize("n", [4, 65, 5000])
+def test_host_build_with_one_huge_triangle(n, far):
+    """One triangle whose box area overflows takes no other out of the tree."""
+    rng = np.random.default_rng(n)
+    t = (rng.random((n, 1, 3)) * 2 - 1 + 0.3 * rng.normal(size=(n, 3, 3))).astype(np.float32)
+    t[n // 3, 0] = (far, -far, far)
+    nodes, tris, depth = reina_rt.bvh_build_host(t.reshape(-1, 9))
+    assert _leaf_counts(nodes).sum() == n and _leaf_counts(nodes).max() <= 3
+    orc = oracle.OracleScene(soup_arrays(t.reshape(-1, 9)), make_desc)   # FP32 nodes: 8 bits do not cover such boxes
+    orc.set_bvh(nodes, tris, 256)
+    o = rng.uniform(-2, 2, (3000, 3)).astype(np.float32)
+    rays = rays_from(o, t[np.arange(1, 3001) % n].mean(1) - o)
+    rays = rays[np.isfinite(rays["dx"])]
+    hb, (hv, _) = orc.brute32(rays), orc.bvh(rays)
+    assert np.array_equal(hb["prim"], hv["prim"]) and np.array_equal(hb["t"], hv["t"])
+    assert (hb["prim"] != 0xFFFFFFFF).mean() > 0.5
+
+
 def decode_quantized(q):
     """(N, 6, 8) float32 decoded child planes of 80-byte quantized nodes, in
     the FP32 node's order lo_x hi_x lo_y hi_y lo_z hi_z. q * s is exact in
