@@ -431,7 +431,7 @@ __device__ __forceinline__ void partition_range(const Task& T, const BinScale& b
         for (int q = 0; q < 12; ++q) {
             const bool is_min = (q % 6) < 3;
             const float v = is_min ? wave_min(sb[sd][q]) : wave_max(sb[sd][q]);
-            if (lane == 0 && v == v && fabsf(v) != INFINITY) {
+            if (lane == 0) {   // also an infinity: a wave without triangles of this side changes nothing
                 if (is_min) atomicMin(&s_side[sd][q], ord_key(v));
                 else atomicMax(&s_side[sd][q], ord_key(v));
             }

@@ -194,3 +194,26 @@ def test_one_huge_triangle_beside_others(cuda, n, far):
     assert float((hits.view(torch.int32)[:, 1] >= 0).float().mean()) > 0.9
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("n", [400, 9000])
+@pytest.mark.parametrize("corner", [3e38, -3e38])
+def test_infinite_box_beside_the_outermost_triangles(cuda, n, corner):
+    """A triangle that reaches to infinity (x = 2^32 times its corner) among
+    the 64 triangles furthest out on that side, which one wave partitions: its
+    boxes hold them all the same."""
+    torch = cuda
+    t = _soup(n, "soup").astype(np.float32)
+    t[:64, :, 0] += np.copysign(np.float32(20.0), np.float32(corner))
+    local = t.copy()
+    local[:, :, 0] *= np.float32(2.0 ** -32)
+    local[10, 0, 0] = corner
+    arrays = _arrays(local)
+    arrays["instances"][0]["transform"][0] = 2.0 ** 32
+    a, b = reina_rt.DeviceScene(arrays), reina_rt.DeviceScene(arrays, flags=abi.BUILD_HOST)
+    _check_tree(a, n)
+    _check_tree(b, n)
+    hits = _same_hits(torch, a, b, _aimed_rays(torch, np.delete(t[:64], 10, 0).mean(1), n))
+    assert float((hits.view(torch.int32)[:, 1] >= 0).float().mean()) > 0.9
+    a.close()
+    b.close()
