@@ -674,11 +674,13 @@ __global__ __launch_bounds__(256) void k_big_emit(const Task* __restrict__ tasks
 }
 
 // Lexicographic (key, payload) bitonic sort across lanes 0..width-1 (width a
-// power of two), ascending.
-__device__ __forceinline__ void wave_sort(float& key, uint32_t& pay, uint32_t lane, uint32_t width) {
+// power of two), ascending. Integer keys: every pair has an order, so the
+// lanes of a pair never keep the same entry. As floats, a NaN compares false
+// either way and both lanes kept one entry of the two.
+__device__ __forceinline__ void wave_sort(uint32_t& key, uint32_t& pay, uint32_t lane, uint32_t width) {
     for (uint32_t k = 2; k <= width; k <<= 1) {
         for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            const float ok = __shfl_xor(key, (int)j);
+            const uint32_t ok = __shfl_xor(key, (int)j);
             const uint32_t op = __shfl_xor(pay, (int)j);
             const bool other_less = ok < key || (ok == key && op < pay);
             const bool up = (lane & k) == 0u || k == width;
@@ -728,10 +730,11 @@ __global__ __launch_bounds__(256) void k_small_tasks(const SmallTask* __restrict
             const float la = a == 0 ? lo.x : a == 1 ? lo.y : lo.z, ha = a == 0 ? hi.x : a == 1 ? hi.y : hi.z;
             // lane k < sz starts with the range's k-th triangle, in lane r0 + k
             const uint32_t from0 = min(r0 + lane, 63u);
-            float key = __shfl(0.5f * la + 0.5f * ha, (int)from0);
-            if (lane >= sz) key = INFINITY;
+            // (+ 0: both zeros have one key)
+            uint32_t key = ord_key(__shfl(0.5f * la + 0.5f * ha, (int)from0) + 0.0f);
+            if (lane >= sz) key = 0xFFFFFFFFu;
             uint32_t pay = from0;
-            if (lane >= sz) pay = 64u + lane;   // after every triangle, also one with an infinite key
+            if (lane >= sz) pay = 64u + lane;   // after every triangle, whatever its key
             wave_sort(key, pay, lane, width);
             if (lane >= sz) pay = lane;
             // lane k (< sz) now holds the k-th range triangle in centroid order

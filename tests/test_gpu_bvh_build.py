@@ -217,3 +217,55 @@ def test_infinite_box_beside_the_outermost_triangles(cuda, n, corner):
     assert float((hits.view(torch.int32)[:, 1] >= 0).float().mean()) > 0.9
     a.close()
     b.close()
+
+
+# the corners of a triangle that is not finite, on the x axis; an infinity is
+# 3e38 under an instance that scales x by 2^32, a NaN reaches every axis. The
+# centroid is NaN for three NaN corners and for -inf beside +inf.
+NON_FINITE = {"nan": (np.nan,) * 3, "negative_nan": (-np.nan,) * 3, "part_nan": (np.nan, 0.0, 2.0 ** -32),
+              "inf": (0.0, 3e38, 2.0 ** -32), "both_inf": (-3e38, 0.0, 3e38), "all_inf": (3e38,) * 3}
+
+
+@pytest.mark.parametrize("kind", list(NON_FINITE) + ["mixed"])
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 33, 64, 65, 129, 5000])
+def test_non_finite_triangles_take_no_other_out(cuda, n, kind):
+    """Triangles that are not finite beside finite ones, several in one wave's
+    sort: every triangle is in one leaf once, and a ray finds the closest
+    finite triangle."""
+    torch = cuda
+    rng = np.random.default_rng(n)
+    t = _soup(n, "soup").astype(np.float32)
+    bad = np.union1d(np.nonzero(rng.random(n) < (0.4 if n < 200 else 0.01))[0], [n // 2])
+    good = np.setdiff1d(np.arange(n), bad)
+    local = t.copy()
+    local[:, :, 0] *= np.float32(2.0 ** -32)
+    for i in bad:
+        local[i, :, 0] = NON_FINITE[list(NON_FINITE)[i % len(NON_FINITE)] if kind == "mixed" else kind]
+    arrays = _arrays(local)
+    arrays["instances"][0]["transform"][0] = 2.0 ** 32
+    dev = reina_rt.DeviceScene(arrays)
+    nodes, tris = dev.export_bvh()
+    tris = tris.reshape(-1, 3, 4)
+    assert np.array_equal(np.sort(tris[:, 0, 3].copy().view(np.uint32)), np.arange(n))
+    assert np.isfinite(tris[:, :, :3]).all((1, 2)).sum() == len(good)
+    nodes = nodes.reshape(-1, 256)
+    first = (nodes[:, 196:200].copy().view(np.uint32) & 0xFFFFFF).astype(int)
+    meta = nodes[:, 200:208].astype(int)
+    leaf = (meta != 0) & (meta < 0x80)
+    slots = [(first + (meta & 31) + j)[leaf & ((meta >> 5) > j)] for j in range(3)]
+    assert np.array_equal(np.sort(np.concatenate(slots)), np.arange(n))
+    if len(good) == 0:
+        dev.close()
+        return
+    ref = reina_rt.DeviceScene(_arrays(t[good]))
+    rays = _aimed_rays(torch, t[good].mean(1), n)
+    h, hr = torch.zeros((4096, 4), device="cuda"), torch.zeros((4096, 4), device="cuda")
+    dev.intersect(rays.data_ptr(), h.data_ptr(), 4096)
+    ref.intersect(rays.data_ptr(), hr.data_ptr(), 4096)
+    torch.cuda.synchronize()
+    prim, pref = (x.view(torch.int32)[:, 1].cpu().numpy() for x in (h, hr))
+    assert (pref >= 0).mean() > 0.9
+    assert np.array_equal(prim, np.where(pref >= 0, good[np.maximum(pref, 0)], -1))
+    assert torch.equal(h[:, 0].view(torch.int32), hr[:, 0].view(torch.int32))
+    dev.close()
+    ref.close()
