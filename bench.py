@@ -10,8 +10,10 @@ value = every traced extension ray (primary + secondary) / wall time of the
 K timed frames, scene already resident in HBM.
 
 roofline: the extend kernel (BVH8 traversal) over the frame's bounce
-iterations; the last few live paths (ReinaTuning.tail_paths) finish in one
-tail launch that is timed separately (tail_ms) and not part of the roofline.
+iterations, in traces of the same frame whose paths move to the tail launch
+when 2^20 are live (ReinaTuning.tail_paths; the launch is timed separately,
+tail_ms, and not part of the roofline). The timed frames use the autotuned
+threshold; at 2^22 they run whole in the tail kernel.
 traffic: HBM bytes per launch of
 that kernel on this workload from the committed rocprofv3 PMC summary
 (profiles/k_trace_icosphere_1080p_64spp.md: FETCH_SIZE x 2 + WRITE_SIZE, scaled by a
@@ -207,7 +209,7 @@ def main():
     if not a.no_roofline:
         out["roofline"] = roofline(dev, frame, NODE_BYTES, torch)
         if (W, H, a.spp, a.depth) == (1920, 1080, 64, 8):
-            tr, tt = profiled_traffic("k_trace_icosphere_1080p_64spp.md", dev.get_tuning())
+            tr, tt = profiled_traffic("k_trace_icosphere_1080p_64spp.md", roofline_tuning(dev.get_tuning()))
             out["roofline"]["traffic"] = tr
             out["roofline"]["traffic_tuning"] = tt
 
@@ -305,6 +307,17 @@ def profiled_traffic(name, tuning):
             return v, t
     return None, None
 
+# The roofline's traces run the extend kernel until this many paths are live.
+ROOFLINE_TAIL = 1 << 20
+
+
+def roofline_tuning(tuning):
+    """The tuning of the roofline's traces: the run's own, with the tail launch
+    at ROOFLINE_TAIL live paths where the run's would come earlier (a 1080p
+    frame runs whole in the tail kernel at 2^22)."""
+    return dict(tuning, tail_paths=min(tuning["tail_paths"], ROOFLINE_TAIL))
+
+
 def profiled_tunings(name):
     """The tunings (dicts of TUNING_KEYS) of the traffic lines in a committed
     rocprofv3 summary."""
@@ -322,11 +335,12 @@ def profiled_tunings(name):
 def run_autotune(dev, sec, sh, torch, frame=None, profile=None):
     """Stage 1 on the secondary batch; stage 2 (when `frame` is given) on
     whole frames: the 3 fastest stage-1 settings and the defaults, each with
-    tail thresholds 2^18 / 2^19 / 2^20, plus the tunings the committed
-    profile `profile` was taken at. Frame times within 1.5% are ties (the
-    spread between runs of one tuning): when the fastest tuning has no
-    profile line, the fastest profiled one among its ties is installed, so
-    the run's extend kernel has a measured HBM traffic figure."""
+    tail thresholds 2^18 / 2^19 / 2^20 / 2^22, plus the launch parameters the
+    committed profile `profile` was taken at, with its own threshold and with
+    2^22. Frame times within 1.5% are ties (the spread between runs of one
+    tuning): when the roofline's traces at the fastest tuning have no profile
+    line, the fastest profiled one among its ties is installed, so that their
+    extend kernel has a measured HBM traffic figure."""
     from reina_rt.autotune import tune_frame, tune_traversal
     d0 = dev.get_tuning()
     cus = torch.cuda.get_device_properties(0).multi_processor_count
@@ -349,19 +363,21 @@ def run_autotune(dev, sec, sh, torch, frame=None, profile=None):
         base["grid_blocks"] = d0["grid_blocks"]
         if base not in top:
             top.append(base)
-        cands = [dict(c, tail_paths=tp) for c in top for tp in (1 << 18, 1 << 19, 1 << 20)]
+        cands = [dict(c, tail_paths=tp) for c in top for tp in (1 << 18, 1 << 19, 1 << 20, 1 << 22)]
         shade = d0["shade_blocks"]
         for t in (profiled_tunings(profile) if profile else []):
             c = {k: t[k] for k in ("stack_depth", "refill_min", "waves_per_simd", "grid_blocks", "tail_paths")}
-            if t["shade_blocks"] == shade and t["stack_depth"] >= d0["stack_depth"] and c not in cands:
-                cands.append(c)
+            for cc in (c, dict(c, tail_paths=1 << 22)):
+                if t["shade_blocks"] == shade and t["stack_depth"] >= d0["stack_depth"] and cc not in cands:
+                    cands.append(cc)
         fwin, ftable = tune_frame(dev, torch, frame, cands)
         out["frame_fastest"] = dict(fwin)
         if profile:
             cur = dev.get_tuning()
-            if profiled_traffic(profile, cur)[0] is None:
+            if profiled_traffic(profile, roofline_tuning(cur))[0] is None:
                 ties = [r for r in ftable if r["ms"] <= fwin["ms"] * 1.015 and
-                        profiled_traffic(profile, dict(cur, **{k: v for k, v in r.items() if k != "ms"}))[0]]
+                        profiled_traffic(profile, roofline_tuning(dict(cur, **{k: v for k, v in r.items()
+                                                                               if k != "ms"})))[0]]
                 if ties:
                     fwin = min(ties, key=lambda r: r["ms"])
                     dev.set_tuning(**{k: v for k, v in fwin.items() if k != "ms"})
@@ -427,13 +443,18 @@ def time_frames(frame, warmup, steps, torch):
 def roofline(dev, frame, node_bytes, torch):
     """Extend-kernel roofline of one frame: algorithmic bytes from the
     counting build, average launch time from HIP events around every extend
-    launch on the trace's stream."""
+    launch on the trace's stream. The frame is traced at roofline_tuning: it
+    is the timed frames' own schedule only where those, too, start in bounce
+    iterations ("timed_tail_paths")."""
     from reina_rt import abi
+    tun = dev.get_tuning()
+    dev.set_tuning(**roofline_tuning(tun))
     dev.set_trace_options(abi.TRACE_COUNT)
     stc = frame(0, dev)
     dev.set_trace_options(abi.TRACE_TIME_EXTEND)
     stt = frame(0, dev)
     dev.set_trace_options(0)
+    dev.set_tuning(**tun)
     torch.cuda.synchronize()
     assert stc.extension_rays == stt.extension_rays and stc.tail_rays == stt.tail_rays
     nrays = stt.extension_rays - stt.tail_rays   # rays traced by k_trace launches (the tail kernel is not counted)
@@ -465,6 +486,8 @@ def roofline(dev, frame, node_bytes, torch):
         "extend_grays_per_s": round(nrays / (stt.extend_ms * 1e-3) / 1e9, 3),
         "tail_rays": int(stt.tail_rays),
         "tail_ms": round(float(stt.tail_ms), 3),
+        "tail_paths": int(roofline_tuning(tun)["tail_paths"]),
+        "timed_tail_paths": int(tun["tail_paths"]),
     }
 
 
@@ -788,7 +811,7 @@ def instanced_block(a, torch):
         if not a.no_roofline:
             res[name]["roofline"] = roofline(d, frame, 80 if name == "quantized" else 208, torch)
             if name == "fp32":
-                tr, tt = profiled_traffic("k_trace_instanced_8m_1080p_32spp.md", d.get_tuning())
+                tr, tt = profiled_traffic("k_trace_instanced_8m_1080p_32spp.md", roofline_tuning(d.get_tuning()))
                 res[name]["roofline"]["traffic"] = tr
                 res[name]["roofline"]["traffic_tuning"] = tt
     if "fp32" in devs and "quantized" in devs:

@@ -346,8 +346,8 @@ int reina_rt_trace_stats(ReinaScene* scene, ReinaTraceStats* out);
 /* Launch parameters of the traversal / shading kernels. Defaults are set at
  * scene creation (stack depth from the BVH depth, refill 32, 8 traversal
  * blocks per CU at stack depth 8 and 4 above, 16 shade blocks per CU, the
- * compiler's register budget, tail launch at 2^20 live paths, claims of 128
- * rays); the autotuner in the Python package searches them per scene. */
+ * compiler's register budget, the tail launch by REINA_RT_TAIL_AUTO, claims of
+ * 128 rays); the autotuner in the Python package searches them per scene. */
 typedef struct ReinaTuning {
     uint32_t stack_depth;   /* LDS stack entries per lane: 8, 16, 24 or 32 (>= BVH depth - 1) */
     uint32_t refill_min;    /* idle lanes per wave that trigger a refill, 1..64                */
@@ -355,12 +355,15 @@ typedef struct ReinaTuning {
     uint32_t shade_blocks;  /* shade blocks (256 threads), a multiple of 8                      */
     uint32_t waves_per_simd;/* traversal register budget: 0 (compiler's choice), 4, 5, 6 or 8      */
     uint32_t tail_paths;    /* when at most this many paths are live, the frame ends in one
-                               tail launch (per-wave extend/shade steps); 0 = never; the
-                               default, 2^20, stands for 2^22 in a trace without next-event
-                               estimation, COUNT or TIME_EXTEND                                */
+                               tail launch (per-wave extend/shade steps); 0 = never;
+                               REINA_RT_TAIL_AUTO (the default)                                */
     uint32_t claim_rays;    /* rays a traversal wave claims from its queue partition with one
                                atomic: 64, 128, 256 or 512 (0 = 128)                           */
 } ReinaTuning;
+/* ReinaTuning.tail_paths: 2^20 in a trace with next-event estimation, COUNT or
+ * TIME_EXTEND and in a server, 2^22 in any other trace. Every other value is
+ * the number itself (a frame has fewer than 2^31 paths). */
+#define REINA_RT_TAIL_AUTO 0xFFFFFFFEu
 int reina_rt_get_tuning(const ReinaScene* scene, ReinaTuning* out);
 int reina_rt_set_tuning(ReinaScene* scene, const ReinaTuning* tuning);
 
@@ -441,8 +444,8 @@ typedef struct ReinaServerDesc {
     uint32_t quantized;          /* node format of every scene served: 0 FP32, 1 8-bit   */
     ReinaTuning tuning;          /* shared-kernel launch parameters; zeros = defaults
                                     (stack_depth bounds the BVH depth of served scenes;
-                                    tail_paths 0 = 2^20, refill_min 0 = 32,
-                                    REINA_RT_TAIL_OFF = never)                           */
+                                    tail_paths 0 or REINA_RT_TAIL_AUTO = 2^20,
+                                    REINA_RT_TAIL_OFF = never, refill_min 0 = 32)        */
     uint32_t flags;              /* REINA_RT_SERVER_NEE or 0                             */
     uint32_t admit_paths;        /* admission stops while this many paths are in flight
                                     in the shared queues (live paths of the last graph +

@@ -421,7 +421,7 @@ int reina_rt_scene_create(const ReinaSceneDesc* d, ReinaScene** out) {
     s->tune.refill_min = 32;
     s->tune.grid = cus * (s->tune.stack_depth <= 8 ? 8 : 4);
     s->tune.shade_grid = cus * 16;   // fills every CU to its register-limited occupancy (latency hiding)
-    s->tune.tail_paths = kDefaultTailPaths;
+    s->tune.tail_paths = REINA_RT_TAIL_AUTO;
     s->min_stack = s->tune.stack_depth;
     *out = s;
     return REINA_RT_OK;
@@ -630,8 +630,9 @@ int reina_rt_trace(ReinaScene* s, const RtPushConsts* pc, float* image, uint32_t
     const uint32_t K = 4;   // iterations between queue-length readbacks
     s->tail_count = 0;
     s->xev_used = 0;
-    const uint32_t tail_paths = s->tune.tail_paths == kDefaultTailPaths && !nee && !timex && !count
-                                    ? kDefaultTailPathsPlain : s->tune.tail_paths;
+    const uint32_t tail_paths = s->tune.tail_paths != REINA_RT_TAIL_AUTO ? s->tune.tail_paths
+                                : nee || timex || count                  ? kDefaultTailPaths
+                                                                         : kDefaultTailPathsPlain;
     while (it < max_iters && live != 0) {
         const uint32_t slot = it % 3, in_q = it & 1u;
         if (live <= tail_paths) {

@@ -25,11 +25,12 @@ int fail(int code, const std::string& msg);
     } while (0)
 
 // Live paths at or below which reina_rt_trace ends the frame in one tail
-// launch (ReinaTuning.tail_paths default).
+// launch where tail_paths is REINA_RT_TAIL_AUTO: with next-event estimation,
+// or the options that count or time the extend kernel, which then has to run
+// (and a server's default) ...
 constexpr uint32_t kDefaultTailPaths = 1u << 20;
-// What the default stands for in a trace without next-event estimation (and
-// without the options that count or time the extend kernel, which then has to
-// run): a frame of up to 2^22 paths is one tail launch from its first ray on.
+// ... and in every other trace: a frame of up to 2^22 paths is one tail launch
+// from its first ray on.
 // The tail keeps a pixel's state and ray in registers, where a bounce
 // iteration moves ~200 bytes per ray through HBM and ends with its slowest
 // waves. ms at 2^20 | 2^22 | 2^24: 1080p 64 spp, 327,686 triangles

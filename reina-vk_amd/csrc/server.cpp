@@ -456,7 +456,7 @@ int reina_rt_server_create(const ReinaServerDesc* d, ReinaServer** out) {
     if ((int)d->device >= ndev) return fail(REINA_RT_ERR_INVALID_ARG, "device ordinal out of range");
     Tuning tu{d->tuning.stack_depth, d->tuning.refill_min, d->tuning.grid_blocks, d->tuning.shade_blocks,
               d->tuning.waves_per_simd, d->tuning.tail_paths};
-    if (tu.tail_paths == 0) tu.tail_paths = kDefaultTailPaths;
+    if (tu.tail_paths == 0 || tu.tail_paths == REINA_RT_TAIL_AUTO) tu.tail_paths = kDefaultTailPaths;
     else if (tu.tail_paths == REINA_RT_TAIL_OFF) tu.tail_paths = 0;   // internally 0 = never
     if (tu.stack_depth == 0) tu.stack_depth = 16;
     if (tu.stack_depth != 8 && tu.stack_depth != 16 && tu.stack_depth != 24 && tu.stack_depth != 32)

@@ -169,6 +169,7 @@ SERVER_BYTES_PER_PIXEL = 152
 SERVER_BYTES_PER_PIXEL_NEE = 216
 SERVER_NEE = 0x1
 TAIL_OFF = 0xFFFFFFFF
+TAIL_AUTO = 0xFFFFFFFE
 REQ_QUEUED, REQ_RUNNING, REQ_DONE, REQ_FAILED = 0, 1, 2, 3
 
 TRACE_TIME_EXTEND = 0x1

@@ -46,3 +46,45 @@ def test_parse_tuning():
     b = _bench()
     assert b.parse_tuning("16,32,2048,4096,4,1048576", "--tuning") == dict(
         stack_depth=16, refill_min=32, grid_blocks=2048, shade_blocks=4096, waves_per_simd=4, tail_paths=1048576)
+
+
+class _FakeStats:
+    extension_rays, tail_rays, node_visits, tri_tests = 1000, 400, 3000, 1500
+    extend_launches, extend_ms, trace_ms, tail_ms = 4, 2.0, 5.0, 1.0
+
+
+class _FakeScene:
+    """What bench.roofline calls on a scene; log: the tail threshold of every trace."""
+
+    def __init__(self, tail_paths):
+        self.tuning = dict(stack_depth=16, refill_min=32, grid_blocks=2048, shade_blocks=4096, waves_per_simd=4,
+                           tail_paths=tail_paths, claim_rays=128)
+        self.log = []
+
+    def get_tuning(self):
+        return dict(self.tuning)
+
+    def set_tuning(self, **kw):
+        self.tuning.update(kw)
+
+    def set_trace_options(self, options):
+        pass
+
+
+def test_roofline_traces_run_the_extend_kernel():
+    """At a threshold above 2^20 (2^22, or the library's choice) the roofline's
+    traces use 2^20 and say so; the run's own tuning is back afterwards."""
+    b = _bench()
+    sys.path.insert(0, os.path.join(ROOT, "reina-vk_amd"))
+    from reina_rt import abi
+    torch_ = type("T", (), {"cuda": type("C", (), {"synchronize": staticmethod(lambda: None)})})
+    for tail, used in ((1 << 22, 1 << 20), (abi.TAIL_AUTO, 1 << 20), (1 << 20, 1 << 20), (1 << 18, 1 << 18)):
+        dev = _FakeScene(tail)
+
+        def frame(batch, d):
+            d.log.append(d.tuning["tail_paths"])
+            return _FakeStats
+        r = b.roofline(dev, frame, 208, torch_)
+        assert dev.log == [used, used] and dev.tuning["tail_paths"] == tail
+        assert r["tail_paths"] == used and r["timed_tail_paths"] == tail
+        assert r["achieved"] is not None
