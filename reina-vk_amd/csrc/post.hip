@@ -21,10 +21,12 @@
 // the percentage, so of the 577 taps of a 1920-pixel row at the default
 // radius only the middle 145 have a weight that FP32 can hold. A zero weight
 // adds nothing to a finite sum; a row or column window holding a non-finite
-// value (zero times which is NaN) sums every tap. 1920x1080, radius 5: blurX
-// 1091 -> 58 us, blurY with combine and tonemap 620 -> 65 us (3.6 G operations
-// of the weighted taps: 46 us each at one per lane and clock); 341x213: 38 ->
-// 16 us.
+// value (zero times which is NaN) sums every tap (add_every_tap). 1920x1080,
+// radius 5: blurX 1091 -> 58 us, blurY with combine and tonemap 620 -> 65 us
+// (3.6 G operations of the weighted taps: 46 us each at one per lane and
+// clock); 341x213: 38 -> 16 us. With a NaN in one row, or in every row, all of
+// it: 1920x1080 1642 -> 167 and 281 us, 1080x1350 974 -> 138 and 203 us,
+// 341x213 41 -> 28 and 31 us.
 // k_blur and k_combine_tonemap, with the taps' weights in LDS, take the sizes
 // those two do not (see launch_postprocess).
 #include <hip/hip_runtime.h>
@@ -163,6 +165,49 @@ __device__ __forceinline__ void add_taps(const Taps& t, int m0, const float (&x)
     }
 }
 
+// Adds every tap of R neighbouring outputs, those without a weight too: a
+// sample that is not finite makes them NaN (zero times which is NaN).
+// load(m, x): samples m..m+U-1 as add_taps numbers them, zero outside the image.
+// Samples that all R outputs take without a weight are one multiply-add per
+// channel, into z: all it can add is zero or NaN.
+template <int R, int U, typename Load>
+__device__ __forceinline__ void add_every_tap(const Taps& t, Load load, float (&c)[R][3]) {
+    const int first = t.half - t.k, last = t.half + t.k;   // the stencil of output 0; output j's is j further
+    float z[3] = {0.0f, 0.0f, 0.0f};
+    for (int m = first & ~(U - 1); m <= last + R - 1; m += U) {
+        float x[3][U];
+        load(m, x);
+        if (m >= first + R - 1 && m + U - 1 <= last) {     // in all R stencils
+            if (m >= 0 && m <= 2 * t.half + R - 1) {
+                add_taps<R, U>(t, m, x, c);
+            } else {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) z[a] = z[a] + x[a][u] * 0.0f;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    const int i = m + u - j;               // tap i - half
+                    if (i < first || i > last) continue;
+                    const float w = i < 0 || i > 2 * t.half ? 0.0f : t.w[kTapPad + i];
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) c[j][a] = c[j][a] + x[a][u] * w;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) c[j][a] = c[j][a] + z[a];
+    }
+}
+
 __device__ __forceinline__ V3 blur_mean(const float (&c)[3], float wsum) {
     return wsum < 0.0001f ? v3(0.0f, 0.0f, 0.0f) : v3(c[0] / wsum, c[1] / wsum, c[2] / wsum);
 }
@@ -215,17 +260,20 @@ __global__ __launch_bounds__(1024) void k_blur_row(const float4* __restrict__ in
                 add_taps<R, U>(t, m, x, c);
             }
         } else {
-            for (int j = 0; j < R; ++j) {
-                for (int32_t i = -t.k; i <= t.k; ++i) {
-                    const int32_t x = (int32_t)(x0 + j) + i;
-                    if (x < 0 || x >= (int32_t)W) continue;
-                    const float w = (i < -t.half || i > t.half) ? 0.0f : t.w[kTapPad + i + t.half];
-                    const float* p = s_row + x + t.half;
-                    c[j][0] = c[j][0] + p[0] * w;
-                    c[j][1] = c[j][1] + p[pitch] * w;
-                    c[j][2] = c[j][2] + p[2 * pitch] * w;
+            add_every_tap<R, 4>(t, [&](int m, float (&x)[3][4]) {
+                const int32_t p = (int32_t)x0 + m;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    if constexpr (R == 4) {   // p and pitch are multiples of 4
+                        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                        if ((uint32_t)p < pitch) v = *reinterpret_cast<const float4*>(s_row + a * pitch + p);
+                        x[a][0] = v.x; x[a][1] = v.y; x[a][2] = v.z; x[a][3] = v.w;
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) x[a][u] = (uint32_t)(p + u) < pitch ? s_row[a * pitch + p + u] : 0.0f;
+                    }
                 }
-            }
+            }, c);
         }
 #pragma unroll
         for (int j = 0; j < R; ++j) {
@@ -258,30 +306,23 @@ __global__ __launch_bounds__(256) void k_blur_column(const float4* __restrict__ 
 #pragma unroll
     for (int j = 0; j < R; ++j) c[j][0] = c[j][1] = c[j][2] = 0.0f;
     const float4* col = blurx + x;
+    const auto load = [&](int m, auto& s) {
+#pragma unroll
+        for (int u = 0; u < (int)(sizeof(s[0]) / sizeof(float)); ++u) {
+            const int32_t y = y0 - t.half + m + u;
+            float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (y >= 0 && y < (int32_t)H) v = col[(uint64_t)(uint32_t)y * W];
+            s[0][u] = v.x; s[1][u] = v.y; s[2][u] = v.z;
+        }
+    };
     if (!every) {
         for (int m = 0; m < 2 * t.half + R; m += U) {
             float s[3][U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int32_t y = y0 - t.half + m + u;
-                float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (y >= 0 && y < (int32_t)H) v = col[(uint64_t)(uint32_t)y * W];
-                s[0][u] = v.x; s[1][u] = v.y; s[2][u] = v.z;
-            }
+            load(m, s);
             add_taps<R, U>(t, m, s, c);
         }
     } else {
-        for (int j = 0; j < R; ++j) {
-            for (int32_t i = -t.k; i <= t.k; ++i) {
-                const int32_t y = y0 + j + i;
-                if (y < 0 || y >= (int32_t)H) continue;
-                const float w = (i < -t.half || i > t.half) ? 0.0f : t.w[kTapPad + i + t.half];
-                const float4 v = col[(uint64_t)(uint32_t)y * W];
-                c[j][0] = c[j][0] + v.x * w;
-                c[j][1] = c[j][1] + v.y * w;
-                c[j][2] = c[j][2] + v.z * w;
-            }
-        }
+        add_every_tap<R, 4>(t, load, c);
     }
 #pragma unroll
     for (int j = 0; j < R; ++j) {
