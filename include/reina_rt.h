@@ -370,7 +370,9 @@ int reina_rt_set_tuning(ReinaScene* scene, const ReinaTuning* tuning);
 /* Closest-hit query for a batch of rays (device pointers): the traceRayEXT
  * of shaders/raytrace/raytrace.rgen.glsl:110-122 as a stand-alone kernel.
  * If counters != NULL (device uint32[2*n]) the per-ray node visits and
- * triangle tests are written there (counting build of the same kernel). */
+ * triangle tests are written there (counting build of the same kernel).
+ * Batches of up to 2^18 rays are traced one ray per lane, without the queue:
+ * of ReinaTuning only stack_depth reaches them. */
 int reina_rt_intersect(ReinaScene* scene, const ReinaRay* rays, ReinaHit* hits,
                        uint32_t n, uint32_t* counters, void* stream);
 

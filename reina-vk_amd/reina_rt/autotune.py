@@ -5,7 +5,9 @@ batch (device buffers) over a grid of (LDS stack depth, refill threshold,
 persistent blocks per CU, register budget in waves per SIMD) with HIP events
 on the given stream, and installs the fastest setting on the scene with
 reina_rt_set_tuning. The stack depth must cover the BVH depth, so candidates
-start at the scene's own default.
+start at the scene's own default. A batch of up to ONCE_RAYS rays is traced
+without the queue, where only the stack depth reaches it: there the other
+settings stay as they are.
 
 Stage 2 (tune_frame) times whole frames through reina_rt_trace for a few
 candidate settings (the best of stage 1, the defaults, each with several
@@ -22,6 +24,9 @@ import time
 import itertools
 
 
+ONCE_RAYS = 1 << 18   # reina_rt_intersect traces up to this many rays in one launch without a queue
+
+
 def tune_traversal(dev, torch, rays_ptr, hits_ptr, n, stream=None, cus=None, reps=3,
                    refills=(8, 16, 32, 64), blocks_per_cu=(4, 8), depths=None, waves=(0, 4, 5, 6, 8)):
     stream = stream or torch.cuda.current_stream()
@@ -31,10 +36,16 @@ def tune_traversal(dev, torch, rays_ptr, hits_ptr, n, stream=None, cus=None, rep
     base = dev.get_tuning()
     if depths is None:
         depths = [d for d in (8, 16, 24, 32) if d >= base["stack_depth"]][:2]
+    own = n <= ONCE_RAYS
+    if own:
+        refills, blocks_per_cu, waves = (base["refill_min"],), (base["grid_blocks"] // cus,), (base["waves_per_simd"],)
+
+    def grid(bpc):
+        return base["grid_blocks"] if own else cus * bpc
     table = []
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     for sd, rf, bpc, wv in itertools.product(depths, refills, blocks_per_cu, waves):
-        dev.set_tuning(stack_depth=sd, refill_min=rf, grid_blocks=cus * bpc, waves_per_simd=wv)
+        dev.set_tuning(stack_depth=sd, refill_min=rf, grid_blocks=grid(bpc), waves_per_simd=wv)
         dev.intersect(rays_ptr, hits_ptr, n, stream=sp)   # warm
         best = None
         for _ in range(reps):
@@ -48,7 +59,7 @@ def tune_traversal(dev, torch, rays_ptr, hits_ptr, n, stream=None, cus=None, rep
                       "ms": round(best, 4)})
     win = min(table, key=lambda r: r["ms"])
     dev.set_tuning(stack_depth=win["stack_depth"], refill_min=win["refill_min"],
-                   grid_blocks=cus * win["blocks_per_cu"], waves_per_simd=win["waves_per_simd"])
+                   grid_blocks=grid(win["blocks_per_cu"]), waves_per_simd=win["waves_per_simd"])
     return win, table
 
 
