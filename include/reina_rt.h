@@ -628,7 +628,7 @@ void reina_rt_gltf_free(ReinaGltfScene* scene);
 /* Diagnostic: evaluates the library's FP32 elementary functions on n inputs
  * (device pointers) so that tests can compare them with the host definitions.
  * fn: 0 sin, 1 cos, 2 log, 3 exp, 4 sqrt, 5 pow(x, y = in2), 6 exp2, 7 1/x,
- * 8 1/sqrt(x). */
+ * 8 1/sqrt(x), 9 a texel's byte x in 0..255 over 255. */
 int reina_rt_debug_math(int fn, const float* in, const float* in2, float* out,
                         uint32_t n, void* stream);
 

@@ -185,6 +185,7 @@ __global__ void k_debug_math(int fn, const float* in, const float* in2, float* o
         case 6: r = exp2f_(x); break;
         case 7: r = inv_(x); break;
         case 8: r = inv_sqrt_(x); break;
+        case 9: r = over255((uint32_t)x); break;
         default: r = __builtin_nanf("");
     }
     out[i] = r;

@@ -137,8 +137,9 @@ RT_D float pow5_(float x) { float x2 = x * x; return (x2 * x2) * x; }
 // cover every input; the device forms below take the inputs whose exponent
 // leaves the intermediate steps normal in 10 and 6, and are as exact: their
 // results equal the compiler's for every float of those ranges (2^-100 to
-// 2^126 for the root, 2^-124 to 2^125 for the inverse: all 1.9 and 2.1
-// billion inputs compared on the device, tests/test_gpu_shading_math.py).
+// 2^126 for the root, 2^-124 to 2^125 for the inverse), and all three functions
+// equal double precision rounded to float for all 2^32 inputs
+// (tests/test_gpu_shading_math.py).
 // For the rest (zero, subnormal, infinite, NaN, negative) the wave branches to
 // the compiler's form: a scalar branch on the ballot, which costs the common
 // case no exec-mask work.

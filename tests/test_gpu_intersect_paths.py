@@ -67,6 +67,25 @@ def test_batches_around_the_limit(cuda, arrays, flags):
     dev.close()
 
 
+@pytest.mark.parametrize("flags", [0, abi.NODES_QUANTIZED], ids=["fp32", "q8"])
+def test_every_stack_depth(cuda, arrays, flags):
+    """The kernels of each LDS stack size on both sides of the limit, plain and
+    counting; at 24 and 32 entries fewer blocks are resident than 2^18 rays
+    launch."""
+    torch = cuda
+    dev = reina_rt.DeviceScene(arrays, flags=flags)
+    rays = _rays(torch, LIMIT + 70001)
+    hits, cnt = _query(torch, dev, rays, count=True)
+    for depth in (8, 16, 24, 32):
+        dev.set_tuning(stack_depth=depth)
+        for n in (1000, LIMIT, LIMIT + 70001):
+            for count in (False, True):
+                h, c = _query(torch, dev, rays[:n], count=count)
+                assert torch.equal(h, hits[:n]), (depth, n)
+                assert c is None or torch.equal(c, cnt[:n]), (depth, n)
+    dev.close()
+
+
 @pytest.mark.parametrize("n", [1000, LIMIT + 9])
 def test_noalloc_replays_in_a_graph(cuda, arrays, n):
     """Both kernels under capture, replayed with eager work between."""

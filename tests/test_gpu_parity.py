@@ -154,27 +154,30 @@ def test_intersect_bitexact_icosphere(cuda, icosphere_arrays):
 
 
 def test_intersect_claims_any_batch_size(cuda, icosphere_arrays):
-    """The traversal kernel's claims give every ray exactly once, whatever the
-    batch size and launch shape: partitions with no rays (fewer rays than
-    partitions), claims that take a partition's last rays exactly or run past
-    its end, and grids far larger than the batch, whose late waves find every
-    partition used up. Hits equal the full batch's (pinned to the oracle by
-    test_intersect_bitexact_icosphere) and, for the small batches, the
-    oracle's brute-force scan."""
+    """Every ray exactly once, whatever the batch size and launch shape. Up to
+    2^18 rays there is no queue and the launch settings change nothing. Above,
+    the traversal kernel's claims: some that take a partition's last rays
+    exactly or run past its end, and grids far larger than the batch, whose
+    late waves find every partition used up (partitions without any rays
+    belong to frames: test_render_partitions_bitexact and the frames of a few
+    pixels). Hits equal the largest batch's and, for its first and last rays,
+    the oracle's brute-force scan."""
     torch = cuda
     arrays, cam = icosphere_arrays
     dev = reina_rt.DeviceScene(arrays)
     orc = oracle.OracleScene(arrays, make_desc)
-    rays = random_rays(70001, -1.5, 1.5, 21)
+    limit = 1 << 18
+    rays = random_rays(limit + 70001, -1.5, 1.5, 21)
     full = gpu_intersect(torch, dev, rays)
-    small = rays[:1025]
-    ref = orc.brute32(small)
-    assert np.array_equal(full["prim"][:1025], ref["prim"])
-    assert np.array_equal(_bits(full["t"][:1025]), _bits(ref["t"]))
+    for part in (slice(0, 1025), slice(len(rays) - 1025, len(rays))):
+        ref = orc.brute32(rays[part])
+        assert np.array_equal(full["prim"][part], ref["prim"])
+        assert np.array_equal(_bits(full["t"][part]), _bits(ref["t"]))
     assert (full["prim"] != 0xFFFFFFFF).sum() > 20000   # the batch hits the sphere
     for grid, claim in ((1, 64), (8, 512), (256, 128), (2048, 64), (4096, 512)):
         dev.set_tuning(grid_blocks=grid, claim_rays=claim)
-        for m in (1, 5, 8, 9, 63, 64, 65, 1023, 1025, 8 * 512 + 3, 70001):
+        for m in (1, 5, 8, 9, 63, 64, 65, 1023, 1025, 8 * 512 + 3, 70001, limit, limit + 1, limit + 8 * 64,
+                  limit + 8 * 512 + 3, limit + 70001):
             h = gpu_intersect(torch, dev, rays[:m])
             assert np.array_equal(_bits(h.view(np.float32).reshape(-1, 4)),
                                   _bits(full[:m].view(np.float32).reshape(-1, 4))), (grid, claim, m)
@@ -867,6 +870,15 @@ def test_intersect_f16_inverses_bitexact(cuda, icosphere_arrays):
     ref = orc.brute32(rays)
     assert np.array_equal(h16["prim"], ref["prim"]) and np.array_equal(_bits(h16["t"]), _bits(ref["t"]))
     assert c16[:, 0].sum() >= c32[:, 0].sum()
+    # more than 2^18 rays: the same through the queue kernel
+    many = np.tile(rays, 4)
+    assert len(many) > 1 << 18
+    dev.set_trace_options(abi.TRACE_F16_INV)
+    hq, cq = gpu_intersect(torch, dev, many, counters=True)
+    hn = gpu_intersect(torch, dev, many)
+    dev.set_trace_options(0)
+    assert np.array_equal(_bits(hq), np.tile(_bits(h32), (4,) + (1,) * (_bits(h32).ndim - 1)))
+    assert np.array_equal(_bits(hn), _bits(hq)) and np.array_equal(cq, np.tile(c16, (4, 1)))
     print("node visits per ray: FP32 inverses %.3f, FP16 inverses %.3f" % (c32[:, 0].mean(), c16[:, 0].mean()))
     q = reina_rt.DeviceScene(arrays, flags=abi.NODES_QUANTIZED)
     q.set_trace_options(abi.TRACE_F16_INV)

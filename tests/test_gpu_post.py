@@ -26,10 +26,11 @@ def _check(torch, img, radius, threshold):
 
 # radius 5: half-widths k from 0 (4 pixels and fewer) past the last tap with a
 # weight (72: images over 480 pixels); 40 on 500 pixels: more taps than the
-# kernel arguments hold; 5300 pixels: rows longer than the staged LDS row
+# kernel arguments hold; 5300 and 5500 pixels at radius 1: the longest rows that
+# fit the 64 KB stage (64,176 bytes) and past it
 @pytest.mark.parametrize("W,H,radius", [(1, 1, 5.0), (3, 2, 5.0), (63, 5, 5.0), (64, 9, 5.0), (65, 33, 0.7),
                                         (257, 31, 5.0), (487, 3, 5.0), (1023, 513, 5.0), (1030, 521, 2.0), (60, 700, 5.0),
-                                        (500, 7, 40.0), (5300, 3, 1.0)])
+                                        (500, 7, 40.0), (5300, 3, 1.0), (5500, 3, 1.0)])
 def test_postprocess_sizes_bitexact(cuda, W, H, radius):
     rng = np.random.default_rng(W * 1000 + H)
     img = (rng.random((H, W, 4)) ** 4 * 4.0 - 0.1).astype(np.float32)

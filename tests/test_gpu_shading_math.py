@@ -1,6 +1,5 @@
 """The shading kernels' shortcuts against what they stand for: roots and
-inverses, whole numbers
-over 255, texel indices without an integer division, the tangent frame left
+inverses, whole numbers over 255, texel indices without an integer division, the tangent frame left
 out where no surface reads it."""
 import numpy as np
 import pytest
@@ -11,8 +10,20 @@ from reina_rt import scenes
 from reina_rt.scene import make_desc
 
 
+@pytest.mark.gpu
+def test_texel_bytes_over_255_are_the_rounded_quotients(cuda):
+    """The device function for every byte, bit for bit."""
+    torch = cuda
+    n = torch.arange(256, device="cuda", dtype=torch.float32)
+    out = torch.zeros_like(n)
+    reina_rt.debug_math(9, n.data_ptr(), None, out.data_ptr(), 256)
+    torch.cuda.synchronize()
+    want = np.arange(256, dtype=np.float32) / np.float32(255.0)
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
 def test_over_255_is_the_rounded_quotient():
-    """n * c corrected by its exact remainder equals n / 255 for every texel
+    """Why the shortcut is exact: n * c corrected by its exact remainder equals n / 255 for every texel
     value (products of two float32 are exact in float64, so each fused
     multiply-add is one float64 expression rounded once)."""
     n = np.arange(256, dtype=np.float32)
@@ -70,3 +81,29 @@ def test_root_and_inverse_are_correctly_rounded(cuda, fn):
     got = out.cpu().numpy()
     same = (got.view(np.uint32) == ref.view(np.uint32)) | (np.isnan(got) & np.isnan(ref))
     assert same.all(), [hex(b) for b in bits[~same][:8]]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fn", [4, 7, 8], ids=["sqrt", "inverse", "inverse_sqrt"])
+def test_root_and_inverse_of_every_float(cuda, fn):
+    """All 2^32 inputs against double precision rounded to float. The double
+    result has more than 2 x 24 + 1 bits, so rounding it again is the correctly
+    rounded root or quotient; 1 / sqrt(x) rounds both steps."""
+    torch = cuda
+    step = 1 << 26
+    out = torch.empty(step, device="cuda")
+    bad = 0
+    for start in range(-(1 << 31), 1 << 31, step):
+        x = torch.arange(start, start + step, device="cuda", dtype=torch.int64).to(torch.int32).view(torch.float32)
+        reina_rt.debug_math(fn, x.data_ptr(), None, out.data_ptr(), step,
+                            stream=torch.cuda.current_stream().cuda_stream)
+        d = x.double()
+        if fn == 4:
+            ref = d.sqrt().float()
+        elif fn == 7:
+            ref = d.reciprocal().float()
+        else:
+            ref = d.sqrt().float().double().reciprocal().float()
+        same = (out.view(torch.int32) == ref.view(torch.int32)) | (torch.isnan(out) & torch.isnan(ref))
+        bad += int((~same).sum())
+    assert bad == 0

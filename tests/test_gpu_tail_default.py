@@ -52,3 +52,29 @@ def test_tail_paths_as_set(cuda, tail, whole):
     dev.trace(push_consts(cam["eye"], cam["center"], cam["fov"], W, H, 2, 3), img.data_ptr(), W, H)
     assert dev.stats().tail_rays == dev.stats().extension_rays
     dev.close()
+
+
+@pytest.mark.parametrize("flags", [0, abi.NODES_QUANTIZED], ids=["fp32", "q8"])
+@pytest.mark.parametrize("nee", [False, True], ids=["plain", "nee"])
+def test_tail_at_every_stack_depth(cuda, flags, nee):
+    """The tail kernel of each LDS stack size, on grids that fit the GPU at
+    once (256 x 256: 256 blocks) and that do not (640 x 480: 1,200), against
+    bounce iterations."""
+    torch = cuda
+    scene, cam = scenes.icosphere(levels=3)
+    dev = reina_rt.DeviceScene(scene.build_arrays(), flags=flags)
+    dev.set_trace_options(abi.TRACE_NEE if nee else 0)
+    for W, H in ((256, 256), (640, 480)):
+        pc = push_consts(cam["eye"], cam["center"], cam["fov"], W, H, 2, 6)
+        ref, img = (torch.zeros((H, W, 4), device="cuda") for _ in range(2))
+        dev.set_tuning(tail_paths=0)
+        dev.trace(pc, ref.data_ptr(), W, H)
+        rays = dev.stats().extension_rays
+        for depth in (8, 16, 24, 32):
+            dev.set_tuning(tail_paths=1 << 30, stack_depth=depth)
+            img.zero_()
+            dev.trace(pc, img.data_ptr(), W, H)
+            st = dev.stats()
+            assert st.tail_rays == st.extension_rays == rays
+            assert torch.equal(img.view(torch.int32), ref.view(torch.int32)), (W, depth)
+    dev.close()
