@@ -214,7 +214,7 @@ static void build_emissive(ReinaScene* s, const ReinaSceneDesc* d, const std::ve
 }
 
 // Everything but the tree; the tree's build fills the ids of the triangles
-// (mesh), and scene_finish what is derived from them.
+// (mesh), and scene_build ends with what is derived from them.
 static int scene_upload(ReinaScene* s, const ReinaSceneDesc* d, const std::vector<InstanceRec>& inst, uint32_t num_tris,
                         DeviceMesh& mesh, float4*& rec) {
     auto al = [](uint64_t x) { return (x + 255) & ~255ull; };
@@ -764,11 +764,16 @@ int reina_rt_set_trace_options(ReinaScene* s, uint32_t options) {
     return REINA_RT_OK;
 }
 
-// Batches of up to 2^18 rays take k_trace_once: every wave is resident at
-// once (4 per SIMD), so nothing is gained from a queue, whose launch needs its
-// counters cleared first and keeps a wave to claims of 128 rays. The rays are
-// spread over about 2,048 waves, two per SIMD: fewer lanes per wave then
-// diverge less. Per query, queue / once (bounce rays, us): icosphere 1,000
+// Batches of up to 2^18 rays take k_trace_once: at stack depths 8 and 16 every
+// wave is resident at once (4 per SIMD), so nothing is gained from a queue,
+// whose launch needs its counters cleared first and keeps a wave to claims of
+// 128 rays. At depths 24 and 32 the stack's LDS (48 and 64 KB per block) leaves
+// 3 and 2 blocks of 4 waves per CU and the largest batches run in two rounds,
+// which still costs no more than the queue (icosphere, queue / once at depth
+// 24: 2^17 rays 151 / 120-127, 2^18 153-156 / 127-130; at depth 32: 2^17 149 /
+// 125-130, 3 x 2^16 149 / 129, 2^18 151-153 / 148-153, on 8-bit nodes 166 /
+// 167). The rays are spread over about 2,048 waves, two per SIMD: fewer lanes
+// per wave then diverge less. Per query, queue / once (bounce rays, us): icosphere 1,000
 // rays 72 / 48, 16,000 94 / 66, 65,536 110 / 76, 150,000 131 / 98, 300,000 137
 // / 138, 600,000 212 / 222; Cornell box 1,000 camera rays 30 / 13; 8-bit nodes,
 // 100,000 triangles: 65,536 89 / 59, 300,000 109 / 111.

@@ -91,11 +91,6 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// Triangle boxes (plo = lo.xyz, phi = hi.xyz), the identity reference order
-// and the scene's box and centroid bounds. At most kPrepBlocks blocks, each
-// adding its bounds with 12 atomics: one set per wave (61,000 atomics on 12
-// words for 327,686 triangles) took 700 us.
-constexpr uint32_t kPrepBlocks = 512;
 // World-space triangles, world = ((c0 x + c1 y) + c2 z) + c3 in the host
 // flattening's operation order, and the instance and primitive of every
 // triangle; w may be null (only the ids). A thread finds its instance by
@@ -134,6 +129,11 @@ __global__ __launch_bounds__(256) void k_flatten(const InstanceRec* __restrict__
     if (bad) sb->nonfinite = 1;
 }
 
+// Triangle boxes (plo = lo.xyz, phi = hi.xyz), the identity reference order
+// and the scene's box and centroid bounds. At most kPrepBlocks blocks, each
+// adding its bounds with 12 atomics: one set per wave (61,000 atomics on 12
+// words for 327,686 triangles) took 700 us.
+constexpr uint32_t kPrepBlocks = 512;
 __global__ __launch_bounds__(256) void k_prep(const float* __restrict__ wtri, uint32_t n, float4* __restrict__ plo,
                                               float4* __restrict__ phi, uint32_t* __restrict__ ref, SceneBounds* sb) {
     __shared__ float s_b[4][12];

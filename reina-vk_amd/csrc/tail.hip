@@ -89,7 +89,9 @@ __device__ __forceinline__ uint32_t tail_claim(Ctrl* ctrl, uint32_t slot, uint32
 //
 // Ready lanes that trigger shading (without NEE): shade_min while the wave has
 // empty lanes. A wave with a pixel in every lane waits for 3/8 more where more
-// blocks wait than the GPU holds (3 on each of 256 CUs): 1080p 64 spp at 32,
+// blocks wait than the GPU holds (3 on each of 256 CUs by the registers; the
+// stack's LDS leaves 2 at stack depth 32 alone, where grids of 513 to 768
+// blocks keep the lower number): 1080p 64 spp at 32,
 // 40, 44, 48, 56 lanes 72.8, 70.8, 70.3, 70.3, 74.4 ms, 1080x1350 7.61, 7.50,
 // 7.38, 7.37, 7.62 ms. With fewer blocks no other wave fills the wait (256x256
 // 1.47 ms at 32, 1.49 at 44), nor in the server's mixed queue (12 requests
