@@ -654,7 +654,8 @@ def served_block(a, torch):
     out["admit_paths"] = a.admit_paths
     res_mix = [(256, 256), (512, 512), (1280, 720), (1920, 1080)]
     # latency choices, fixed: tail launch at 2^20 live paths beside the loop, admission points every 6
-    # iterations (a sweep at 50-400 requests/s gave p50 and p99 below plain's at every rate with these)
+    # iterations (a sweep at 50-400 requests/s, while plain's 1080p frames began as bounce iterations,
+    # gave p50 and p99 below plain's at every rate with these)
     base = dict(path_budget_bytes=SERVER_BUDGET, tail_paths=1 << 20, graph_iters=6)
     if not a.no_autotune:
         from reina_rt import autotune

@@ -98,7 +98,7 @@ struct Tuning {
     uint32_t grid;          // persistent blocks of 256 threads
     uint32_t shade_grid;    // blocks of the shade kernel
     uint32_t waves_per_simd;  // register budget of the traversal kernel: 0 (compiler's choice), 4, 5, 6 or 8
-    uint32_t tail_paths;      // live paths at which the frame ends in one tail launch (0: never)
+    uint32_t tail_paths;      // live paths at which the frame ends in one tail launch (0: never; a scene's may be REINA_RT_TAIL_AUTO)
     uint32_t claim = 128;     // rays a traversal wave claims with one atomic: 64, 128, 256 or 512
 };
 
